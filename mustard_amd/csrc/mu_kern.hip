@@ -12,14 +12,14 @@ namespace mu {
 
 __global__ MU_GEMM_KERNEL void k_unit_gemm(UnitDesc d)
 {
-    __shared__ double smem[LDS_GEMM];
+    __shared__ __align__(16) double smem[LDS_GEMM];
     run_gemm_item(d, blockIdx.x, smem);
 }
 
 __global__ MU_GEMM_KERNEL void k_batch_gemm(const UnitDesc *units, const uint32_t *item_unit,
                                             const uint32_t *items)
 {
-    __shared__ double smem[LDS_GEMM];
+    __shared__ __align__(16) double smem[LDS_GEMM];
     const uint32_t item = items[blockIdx.x];
     // a private copy of the descriptor lives in registers; a reference into
     // global memory would be re-read after every barrier of the item body
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_batch_gemm_narrow(const UnitDesc
                                                                   const uint32_t *item_unit,
                                                                   const uint32_t *items)
 {
-    __shared__ double smem[LDS_GEMM];
+    __shared__ double smem[LDS_NARROW];
     const uint32_t item = items[blockIdx.x];
     const UnitDesc d = units[item_unit[item]];
     run_gemm_narrow_item(d, (int)(item - d.item_base), smem);

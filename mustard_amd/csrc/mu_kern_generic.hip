@@ -11,7 +11,7 @@ namespace mu {
 
 __global__ __launch_bounds__(WG_THREADS) void k_unit(UnitDesc d)
 {
-    __shared__ double smem[LDS_DOUBLES];
+    __shared__ __align__(16) double smem[LDS_DOUBLES];
     run_item(d, blockIdx.x, smem);
 }
 
@@ -20,7 +20,7 @@ __global__ __launch_bounds__(WG_THREADS) void k_batch(const UnitDesc *units,
                                                       const uint32_t *item_unit,
                                                       const uint32_t *items)
 {
-    __shared__ double smem[LDS_DOUBLES];
+    __shared__ __align__(16) double smem[LDS_DOUBLES];
     const uint32_t item = items[blockIdx.x];
     // a private copy of the descriptor lives in registers; a reference into
     // global memory would be re-read after every barrier of the item body

@@ -55,9 +55,13 @@ __device__ __forceinline__ v4d mfma_f64(double a, double b, v4d c)
 // GEMM / SYRK output block: C[i0:i0+64, j0:j0+64] = beta C + alpha op(A) op(B)
 // ---------------------------------------------------------------------------
 // Four waves in a 2 x 2 grid, each owning a 32 x 32 sub-block (2 x 2 MFMA
-// tiles).  K runs in blocks of 8, double-buffered in LDS.  The kernel that
-// runs GEMM-only batches needs 20 KB of LDS and at most 128 VGPRs per lane,
-// so four workgroups share a CU and their waves hide each other's latency.
+// tiles).  Two bodies: gemm_block_dma for every block of a unit with m, n >=
+// 64 and k >= 16 (gemm_dma_ok), gemm_block for the smaller ones, whose edges
+// it masks; both sum an element over k in the same order, so a result does
+// not depend on which one ran.
+//
+// gemm_block: K runs in blocks of 8, double-buffered in LDS, through
+// registers.
 //
 // LDS layouts.  An operand whose stored columns run along the output
 // dimension ("i-contiguous": A, or B^T) is kept as S[k][i] with a pitch of
@@ -73,27 +77,17 @@ constexpr int LDS_K = GEMM_BM * PK;   // doubles per k-contiguous buffer
 // into the operand; the values that fall outside it are zeroed only when the
 // registers are written to LDS.  With no branch around a load and no use of
 // its result before the LDS store, the compiler's wait counting stays exact
-// and a prefetch stays in flight until the half-step that stores it.  VEC
-// (16-byte aligned operands, even leading dimensions and even m, n, k, set by
-// the lowering) loads element pairs, which then never straddle an edge.
+// and a prefetch stays in flight until the half-step that stores it.
 
 // i-contiguous operand: element (r, k) at p[r + k*ld], r < rows, k < kcols.
 // Thread t covers rows 2(t%32), 2(t%32)+1 of column t/32.
-template <bool VEC>
 __device__ __forceinline__ void ld_icontig(double (&v)[2], const MU_G double *p, int ld, int rows,
                                            int kcols)
 {
     const int t = threadIdx.x, r = (t & 31) * 2, c = t >> 5;
     const int cc = max(0, min(c, kcols - 1));
-    if (VEC) {
-        const int rr = max(0, min(r, rows - 2));
-        const v2d x = *reinterpret_cast<const MU_G v2d *>(p + rr + (size_t)cc * ld);
-        v[0] = x[0];
-        v[1] = x[1];
-    } else {
-        v[0] = p[min(r, rows - 1) + (size_t)cc * ld];
-        v[1] = p[min(r + 1, rows - 1) + (size_t)cc * ld];
-    }
+    v[0] = p[min(r, rows - 1) + (size_t)cc * ld];
+    v[1] = p[min(r + 1, rows - 1) + (size_t)cc * ld];
 }
 
 __device__ __forceinline__ void st_icontig(double *S, const double (&v)[2], int rows, int kcols)
@@ -108,21 +102,13 @@ __device__ __forceinline__ void st_icontig(double *S, const double (&v)[2], int 
 
 // k-contiguous operand: element (r, k) at p[k + r*ld].
 // Thread t covers k = 2(t%4), 2(t%4)+1 of row t/4.
-template <bool VEC>
 __device__ __forceinline__ void ld_kcontig(double (&v)[2], const MU_G double *p, int ld, int rows,
                                            int kcols)
 {
     const int t = threadIdx.x, k = (t & 3) * 2, r = t >> 2;
     const int rr = min(r, rows - 1);
-    if (VEC) {
-        const int kk = max(0, min(k, kcols - 2));
-        const v2d x = *reinterpret_cast<const MU_G v2d *>(p + kk + (size_t)rr * ld);
-        v[0] = x[0];
-        v[1] = x[1];
-    } else {
-        v[0] = p[max(0, min(k, kcols - 1)) + (size_t)rr * ld];
-        v[1] = p[max(0, min(k + 1, kcols - 1)) + (size_t)rr * ld];
-    }
+    v[0] = p[max(0, min(k, kcols - 1)) + (size_t)rr * ld];
+    v[1] = p[max(0, min(k + 1, kcols - 1)) + (size_t)rr * ld];
 }
 
 __device__ __forceinline__ void st_kcontig(double *S, const double (&v)[2], int rows, int kcols)
@@ -147,7 +133,7 @@ __device__ __forceinline__ double frag_b(const double *S, int k, int j)
     return TB ? S[k * PI + j] : S[j * PK + k];
 }
 
-template <bool TA, bool TB, bool VEC>
+template <bool TA, bool TB>
 __device__ __attribute__((always_inline)) inline void gemm_block(const UnitDesc &u, int bi, int bj, bool lower_only, double *smem)
 {
     constexpr int BM = GEMM_BM, BN = GEMM_BN, BK = GEMM_BK;
@@ -178,13 +164,13 @@ __device__ __attribute__((always_inline)) inline void gemm_block(const UnitDesc 
         // a block past K is read (and zeroed) at k-offset 0, inside the operand
         const int kc = K - k0, ks = kc > 0 ? k0 : 0;
         if (TA)
-            ld_kcontig<VEC>(ra, A + ks, u.lda, rows, kc);
+            ld_kcontig(ra, A + ks, u.lda, rows, kc);
         else
-            ld_icontig<VEC>(ra, A + (size_t)ks * u.lda, u.lda, rows, kc);
+            ld_icontig(ra, A + (size_t)ks * u.lda, u.lda, rows, kc);
         if (TB)
-            ld_icontig<VEC>(rb, B + (size_t)ks * u.ldb, u.ldb, cols, kc);
+            ld_icontig(rb, B + (size_t)ks * u.ldb, u.ldb, cols, kc);
         else
-            ld_kcontig<VEC>(rb, B + ks, u.ldb, cols, kc);
+            ld_kcontig(rb, B + ks, u.ldb, cols, kc);
     };
     // store the block loaded for k-offset k0 (zeroing what lies outside)
     auto store = [&](const double (&ra)[2], const double (&rb)[2], double *As, double *Bs,
@@ -273,6 +259,229 @@ epilogue:
                     gp(u.c)[(i0 + r) + (size_t)(j0 + c) * u.ldc] =
                         beta * cv[x][y][e] + alpha * acc[x][y][e];
             }
+}
+
+// ---------------------------------------------------------------------------
+// GEMM / SYRK output block, operands copied straight into LDS.
+//
+// What bounds it: the FP64 matrix pipe, and on gfx950 the vector ALU shares
+// it -- every VALU instruction of the k-loop takes about 4 cycles from the
+// MFMAs (a loop of MFMAs and nothing else: adding 8 v_add per MFMA takes 30 %
+// more time, with four waves per SIMD to overlap them).  So the loop below has
+// no masks, no address arithmetic beyond two pointer increments and no
+// staging registers: a k-slice of 16 is copied by four 16-byte-per-lane
+// global_load_lds per wave, the fragments are read at constant offsets, and
+// 16 MFMAs follow; the next slice's copy is in flight meanwhile (two
+// buffers, 32 KB, so up to five workgroups share a CU).  Stand-alone, merged
+// LU update 22000 x 22000 x 1000, lda 24000: 70.9 TFLOP/s, 90 % of the FP64
+// MFMA peak, against 58.6 for the masked loop through registers
+// (gemm_block); 128 x 64 and 128 x 128 blocks in the same form 67.3 and 66.3
+// (fewer waves to cover the barriers).
+//
+// No edges: a block that would pass the last row or column is moved back to
+// end there (needs m, n >= 64) and stores only the part no other block
+// owns, so every load is inside the operand.  The last k % 16 columns go
+// through registers with zeroed padding.  global_load_lds needs only 4-byte
+// alignment, so odd leading dimensions and offsets take this path too.
+//
+// LDS.  An operand contiguous along the output dimension keeps rows of 64
+// (S[k][i], 512 bytes): a lane reads rows i = 2 li, 2 li + 1 of a k with one
+// 16-byte load, which feed its two MFMA tiles, so tile x's index li stands
+// for i = 2 li + x.  An operand contiguous along k keeps 16 k per output
+// index (128 bytes) in 16-byte chunks, chunk c of output o at c ^ ((o / 2) %
+// 8), which makes the 16 outputs of a fragment hit 64 different banks; the
+// copy applies the permutation by choosing which chunk each lane fetches.
+// Operands enter the MFMA swapped (D = op(B)^T op(A)^T), so a lane holds
+// consecutive rows of C: 256-byte runs instead of 32-byte ones.
+// ---------------------------------------------------------------------------
+#define MU_LDS __attribute__((address_space(3)))
+typedef double v2du __attribute__((ext_vector_type(2), aligned(8)));  // C pairs, any alignment
+constexpr int DMA_BK = 16;
+constexpr int DMA_OP = GEMM_BM * DMA_BK;  // doubles per operand buffer
+constexpr int LDS_GEMM_DMA = 4 * DMA_OP;  // 2 operands x 2 buffers (32 KB)
+
+// Units every block of which gemm_block_dma can run (the per-lane byte
+// offsets of a 64-row slice are 32-bit).
+__device__ __forceinline__ bool gemm_dma_ok(const UnitDesc &u)
+{
+    return u.m >= GEMM_BM && u.n >= GEMM_BN && u.k >= DMA_BK && u.lda < (1 << 22) &&
+           u.ldb < (1 << 22);
+}
+
+template <bool TA, bool TB>
+__device__ __attribute__((always_inline)) inline void gemm_block_dma(const UnitDesc &u, int bi,
+                                                                     int bj, bool lower_only,
+                                                                     double *smem)
+{
+    constexpr int BM = GEMM_BM, BK = DMA_BK;
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 1, wn = wave >> 1;  // 2 x 2 waves of 32 x 32
+    // block origin, moved back to stay inside; rows < ri and columns < rj of
+    // the moved block belong to its neighbours
+    const int i0 = min(bi * BM, u.m - BM), j0 = min(bj * BM, u.n - BM);
+    const int ri = bi * BM - i0, rj = bj * BM - j0;
+    const int K = u.k, nk = K / BK;
+    const size_t lda = u.lda, ldb = u.ldb;
+    const MU_G char *ap = (const MU_G char *)(gp(u.a) + (TA ? (size_t)i0 * lda : (size_t)i0));
+    const MU_G char *bp = (const MU_G char *)(gp(u.b) + (TB ? (size_t)j0 : (size_t)j0 * ldb));
+    const size_t da = 8 * (TA ? (size_t)BK : BK * lda), db = 8 * (TB ? BK * ldb : (size_t)BK);
+
+    // byte offset of the 16 bytes this lane copies in its wave's copy q (two
+    // per operand): LDS slot s, in order
+    auto slot_off = [&](int q, bool kcontig, size_t ld) -> unsigned {
+        const int s = (wave * 2 + q) * 64 + lane;
+        if (kcontig) {
+            const int o = s >> 3, c = (s & 7) ^ ((o >> 1) & 7);
+            return 8u * ((unsigned)o * (unsigned)ld + 2u * c);
+        }
+        return 8u * ((unsigned)(s >> 5) * (unsigned)ld + 2u * (s & 31));
+    };
+    const unsigned oa0 = slot_off(0, TA, lda), oa1 = slot_off(1, TA, lda);
+    const unsigned ob0 = slot_off(0, !TB, ldb), ob1 = slot_off(1, !TB, ldb);
+    auto copy16 = [&](const MU_G char *p, double *l) {
+        __builtin_amdgcn_global_load_lds((const MU_G unsigned *)p, (MU_LDS unsigned *)l, 16, 0, 0);
+    };
+    auto load = [&](int buf) {
+        double *as = smem + buf * 2 * DMA_OP + wave * 256, *bs = as + DMA_OP;
+        copy16(ap + oa0, as);
+        copy16(ap + oa1, as + 128);
+        copy16(bp + ob0, bs);
+        copy16(bp + ob1, bs + 128);
+        ap += da;
+        bp += db;
+    };
+
+    v4d acc[2][2];
+#pragma unroll
+    for (int x = 0; x < 2; x++)
+#pragma unroll
+        for (int y = 0; y < 2; y++)
+            acc[x][y] = v4d{0.0, 0.0, 0.0, 0.0};
+    // LDS element offset of this lane's fragment of k-step 4 s + lk in an
+    // operand buffer, for a wave whose 32 outputs start at o0
+    auto frag_off = [&](int s, int o0, bool kcontig) -> int {
+        const int o = o0 + li;
+        return kcontig ? o * BK + (((2 * s + (lk >> 1)) ^ ((o >> 1) & 7)) << 1) + (lk & 1)
+                       : (4 * s + lk) * BM + o0 + 2 * li;
+    };
+    int la[4], lb[4];
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        la[s] = frag_off(s, wm * 32, TA);
+        lb[s] = frag_off(s, wn * 32, !TB);
+    }
+    auto compute = [&](int buf) {
+        const double *as = smem + buf * 2 * DMA_OP, *bs = as + DMA_OP;
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            v2d fa, fb;
+            if (TA)
+                fa = v2d{as[la[s]], as[la[s] + 16 * BK]};
+            else
+                fa = *reinterpret_cast<const v2d *>(as + la[s]);
+            if (TB)
+                fb = *reinterpret_cast<const v2d *>(bs + lb[s]);
+            else
+                fb = v2d{bs[lb[s]], bs[lb[s] + 16 * BK]};
+#pragma unroll
+            for (int x = 0; x < 2; x++)
+#pragma unroll
+                for (int y = 0; y < 2; y++)
+                    acc[x][y] = mfma_f64(fb[y], fa[x], acc[x][y]);
+        }
+    };
+    // this wave's copies have landed and every wave has read the other buffer
+    auto sync = [] { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+
+    load(0);
+    int kb = 0;
+    for (; kb + 2 < nk; kb += 2) {
+        sync();
+        load(1);
+        compute(0);
+        sync();
+        load(0);
+        compute(1);
+    }
+    sync();
+    if (kb + 1 < nk) {
+        load(1);
+        compute(0);
+        sync();
+        compute(1);
+    } else {
+        compute(0);
+    }
+    if (const int kt = K - nk * BK) {
+        // the last kt columns into the buffer the last compute left alone
+        double *as = smem + (nk & 1) * 2 * DMA_OP, *bs = as + DMA_OP;
+        auto tail = [&](double *D, const MU_G char *p, bool kcontig, size_t ld) {
+            const MU_G double *g = (const MU_G double *)p;
+#pragma unroll
+            for (int q = 0; q < DMA_OP / WG_THREADS; q++) {
+                const int s = tid + WG_THREADS * q;
+                const int o = kcontig ? s >> 4 : s & 63, k = kcontig ? s & 15 : s >> 6;
+                const size_t kc = min(k, kt - 1);
+                const double v = g[kcontig ? kc + o * ld : o + kc * ld];
+                D[kcontig ? o * BK + (((k >> 1) ^ ((o >> 1) & 7)) << 1) + (k & 1) : s] =
+                    k < kt ? v : 0.0;
+            }
+        };
+        tail(as, ap, TA, lda);
+        tail(bs, bp, !TB, ldb);
+        sync();
+        if (nk & 1)
+            compute(1);
+        else
+            compute(0);
+    }
+
+    // acc[x][y][e]: row r(x) of the block, column c(y, e)
+    const double alpha = u.alpha, beta = u.beta;
+    const size_t ldc = u.ldc;
+    MU_G double *cb = gp(u.c) + i0 + (size_t)j0 * ldc;
+    const int r0 = wm * 32 + (TA ? li : 2 * li), dr = TA ? 16 : 1;
+    auto col = [&](int y, int e) {
+        return wn * 32 + (TB ? 2 * (4 * e + lk) + y : 16 * y + 4 * e + lk);
+    };
+    if (!TA && ri == 0 && rj == 0 && !lower_only) {
+        v2d cv[2][4];
+#pragma unroll
+        for (int y = 0; y < 2; y++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                cv[y][e] = beta != 0.0 ? *(const MU_G v2du *)(cb + r0 + col(y, e) * ldc)
+                                       : v2d{0.0, 0.0};
+#pragma unroll
+        for (int y = 0; y < 2; y++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                *(MU_G v2du *)(cb + r0 + col(y, e) * ldc) =
+                    v2d{beta * cv[y][e][0] + alpha * acc[0][y][e],
+                        beta * cv[y][e][1] + alpha * acc[1][y][e]};
+        return;
+    }
+#pragma unroll
+    for (int x = 0; x < 2; x++) {
+        const int r = r0 + x * dr;
+        double cv[2][4];
+        bool ok[2][4];
+#pragma unroll
+        for (int y = 0; y < 2; y++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int c = col(y, e);
+                ok[y][e] = r >= ri && c >= rj && (!lower_only || i0 + r >= j0 + c);
+                cv[y][e] = (ok[y][e] && beta != 0.0) ? cb[r + c * ldc] : 0.0;
+            }
+#pragma unroll
+        for (int y = 0; y < 2; y++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (ok[y][e])
+                    cb[r + col(y, e) * ldc] = beta * cv[y][e] + alpha * acc[x][y][e];
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1285,7 +1494,9 @@ __device__ __attribute__((always_inline)) inline void factor_small_blk(const Uni
 }
 
 // LDS (doubles) one workgroup needs for any item.
-constexpr int LDS_GEMM = 2 * (LDS_I > LDS_K ? LDS_I : LDS_K) * 2;  // 2 operands x 2 buffers
+constexpr int LDS_GEMM = LDS_GEMM_DMA;
+static_assert(2 * (LDS_I > LDS_K ? LDS_I : LDS_K) * 2 <= LDS_GEMM, "gemm_block: 2 operands x 2 buffers");
+constexpr int LDS_NARROW = 4 * 4 * 4 * 64 / 2 + 1;  // the narrow GEMMs' partial tiles and a flag
 constexpr int LDS_TRSM = TRSM_NMAX * 16 + 16 * 17;
 constexpr int LDS_SMALL = LDS_SMALL_BLK;
 static_assert(TRINV_BLOCKS * 16 * 17 <= LDS_TRSM, "TRINV staging fits the generic LDS");
@@ -1369,10 +1580,10 @@ __device__ __forceinline__ void gemm_dispatch_vec(const UnitDesc &u, int bi, int
             }
         }
 #undef MU_LOW_CASE
-    } else if (u.flags & F_VEC) {
-        gemm_block<TA, TB, true>(u, bi, bj, lo, smem);
+    } else if (gemm_dma_ok(u)) {
+        gemm_block_dma<TA, TB>(u, bi, bj, lo, smem);
     } else {
-        gemm_block<TA, TB, false>(u, bi, bj, lo, smem);
+        gemm_block<TA, TB>(u, bi, bj, lo, smem);
     }
 }
 
@@ -1474,7 +1685,7 @@ __device__ __attribute__((always_inline)) inline void gemm_narrow(const UnitDesc
         }
     }
 }
-static_assert(3 * 4 * 64 <= LDS_GEMM, "narrow GEMM reduction fits the GEMM LDS");
+static_assert(3 * 4 * 64 <= LDS_NARROW, "narrow GEMM reduction fits");
 
 // ---------------------------------------------------------------------------
 // Narrow GEMM with an FP32 A (F_NARROW | F_A32): C = beta C + alpha A B for
@@ -1651,7 +1862,8 @@ __device__ __attribute__((always_inline)) inline void gemm_narrow_a32(const Unit
     if (threadIdx.x == 0)
         __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-static_assert(4 * 4 * 4 * 64 + 1 <= 2 * LDS_GEMM, "FP32-A narrow reduction fits the GEMM LDS");
+static_assert(4 * 4 * 4 * 64 + 1 <= 2 * LDS_NARROW && LDS_NARROW <= LDS_GEMM,
+              "FP32-A narrow reduction fits");
 
 // Narrow GEMM item (F_NARROW units only; kept out of run_gemm_item so the
 // 64 x 64 block kernels keep their register budget).

@@ -86,7 +86,7 @@ static_assert(LDS_PERSIST >= LDS_SMALL, "persistent LDS holds the small factoriz
 
 // The kernel's LDS, at file scope so the item bodies below address it as LDS
 // without a pointer argument.
-__shared__ double p_smem[LDS_PERSIST];
+__shared__ __align__(16) double p_smem[LDS_PERSIST];
 
 // One function per item kind, each kept out of line: its registers are
 // allocated for that body alone, and nothing of it is hoisted into the
