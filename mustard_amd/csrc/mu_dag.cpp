@@ -380,7 +380,10 @@ struct Builder {
                 d.flags |= F_VEC;
             if (kvec(op.flags, op.a, op.lda, op.b, op.ldb, op.k))
                 d.flags |= F_KVEC;
-            d.grp = o.gemm_group > 1 ? o.gemm_group : 1;
+            // grouped only where enough items remain: the updates on the way to
+            // the next panel (2 x 2 blocks inside a nested factorization) are a
+            // chain, and a group of them would run one block after another
+            d.grp = o.gemm_group > 1 && d.gm * d.gn >= 64 ? o.gemm_group : 1;
             int u = add_unit(d);
             f.src = {u};
             f.snk = {u};

@@ -10,6 +10,7 @@
 // worker loop are in mu_sched.hpp; this file binds them to gfx950 atomics,
 // LDS and barriers, and holds the item dispatch.
 #include <algorithm>
+#include <cstddef>
 
 #include "mu_kernels.hpp"
 #include "mu_ops.hpp"
@@ -20,6 +21,8 @@ namespace mu {
 #define AGENT __HIP_MEMORY_SCOPE_AGENT
 
 // Per-lane memory operations at agent scope (the whole GPU: all eight XCDs).
+static_assert(NPRIO == 4 && offsetof(SchedState, done) == 16 && offsetof(SchedState, abort) == 20,
+              "peek reads words 0..5");
 struct DevAtom {
     static __device__ __forceinline__ bool lane0() { return (threadIdx.x & 63) == 0; }
     static __device__ __forceinline__ uint32_t bcast(uint32_t v)
@@ -29,6 +32,18 @@ struct DevAtom {
     static __device__ __forceinline__ uint32_t load(uint32_t *p)
     {
         return __hip_atomic_load(p, __ATOMIC_RELAXED, AGENT);
+    }
+    // the six words at the head of the state, one per lane in one load
+    static __device__ __forceinline__ SchedPeek peek(SchedState *st)
+    {
+        const int l = threadIdx.x & 63;
+        const int v = (int)load(reinterpret_cast<uint32_t *>(st) + (l < 5 ? l : 5));
+        SchedPeek r;
+        for (int p = 0; p < NPRIO; p++)
+            r.cnt[p] = __builtin_amdgcn_readlane(v, p);
+        r.done = (uint32_t)__builtin_amdgcn_readlane(v, 4);
+        r.abort = (uint32_t)__builtin_amdgcn_readlane(v, 5);
+        return r;
     }
     static __device__ __forceinline__ uint32_t load_acquire(uint32_t *p)
     {

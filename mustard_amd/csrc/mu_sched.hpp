@@ -109,13 +109,27 @@ MU_HD void sched_abort(const ExecView &ev, uint32_t code)
     w_store<AT>(&ev.st->abort, 1u);
 }
 
-// The run was aborted, by the device watchdog or by the host.
+// The host's abort word lives in pinned host memory, a PCIe round trip away,
+// so no worker reads it on its way to an item: a waiting worker reads it on
+// every SCHED_HOST_POLLS-th poll (about once a millisecond; with 512 workers
+// polling it every time, an order-6000 LU took 147 ms, most of it waiting
+// behind these reads), a busy one on every 256th item.
+constexpr uint32_t SCHED_HOST_POLLS = 1024;
+
 template <class AT>
-MU_HD bool sched_stopped(const ExecView &ev)
+MU_HD bool sched_host_stopped(const ExecView &ev)
+{
+    return ev.host_abort && AT::bcast(AT::load_system(ev.host_abort)) != 0;
+}
+
+// The run was aborted, by the device watchdog or by the host (the latter
+// looked at every SCHED_HOST_POLLS calls, which `polls` counts).
+template <class AT>
+MU_HD bool sched_stopped(const ExecView &ev, uint32_t &polls)
 {
     if (w_load<AT>(&ev.st->abort))
         return true;
-    return ev.host_abort && AT::bcast(AT::load_system(ev.host_abort)) != 0;
+    return (++polls & (SCHED_HOST_POLLS - 1)) == 0 && sched_host_stopped<AT>(ev);
 }
 
 // Queue all items of unit u on its priority ring (one thread).
@@ -135,23 +149,26 @@ MU_HD void sched_push_unit(const ExecView &ev, uint32_t u)
 }
 
 // Next item for this workgroup (wave-collective), or -1 when the run is
-// over or aborted.  Rings are tried in priority order.  The fast path (an
-// item is queued) reads only the ring counters; the abort words -- one of
-// them in host memory, a PCIe round trip away -- are read on every 16th call
-// (`calls` counts them for the caller) and whenever nothing is queued.
+// over or aborted.  Rings are tried in priority order.  One load of the wave
+// brings the four ring counts, the progress counter and the abort word, so
+// a poll is one memory round trip and an item of any priority is seen by it.
+// `calls` counts the calls of this workgroup.
 template <class AT>
 MU_HD int sched_pop(const ExecView &ev, uint32_t &calls)
 {
-    if ((calls++ & 15u) == 0 && sched_stopped<AT>(ev))
+    if ((++calls & 255u) == 0 && sched_host_stopped<AT>(ev))
         return -1;
     uint64_t t0 = 0, idle = 0;
-    uint32_t seen = 0;
+    uint32_t seen = 0, polls = 0;
     bool first = true;
     for (;;) {
+        const SchedPeek s = AT::peek(ev.st);
+        if (s.abort)
+            return -1;
         for (int p = 0; p < NPRIO; p++) {
-            uint32_t *cnt = reinterpret_cast<uint32_t *>(&ev.st->cnt[p]);
-            if ((int32_t)w_load<AT>(cnt) <= 0)
+            if (s.cnt[p] <= 0)
                 continue;
+            uint32_t *cnt = reinterpret_cast<uint32_t *>(&ev.st->cnt[p]);
             if ((int32_t)w_add<AT>(cnt, 0xffffffffu) <= 0) {
                 w_add<AT>(cnt, 1u);  // none left after all: give the unit back
                 continue;
@@ -166,21 +183,20 @@ MU_HD int sched_pop(const ExecView &ev, uint32_t &calls)
                 const uint32_t v = w_load_acquire<AT>(ev.slots[p] + pos);
                 if (v)
                     return (int)(v - 1);
-                if (sched_stopped<AT>(ev))
+                if (sched_stopped<AT>(ev, polls))
                     return -1;
                 AT::pause();
             }
         }
-        // nothing queued: stop, finish, or wait with the watchdog armed
-        if (sched_stopped<AT>(ev))
+        // nothing queued: finish, stop, or wait with the watchdog armed
+        if (s.done >= ev.nitems)
             return -1;
-        const uint32_t d = w_load<AT>(&ev.st->done);
-        if (d >= ev.nitems)
+        if ((++polls & (SCHED_HOST_POLLS - 1)) == 0 && sched_host_stopped<AT>(ev))
             return -1;
         const uint64_t now = AT::now();
-        if (first || d != seen) {
+        if (first || s.done != seen) {
             first = false;
-            seen = d;
+            seen = s.done;
             t0 = now;
             idle = 0;
         } else if (now - t0 > ev.timeout_ticks) {
@@ -209,6 +225,7 @@ MU_HD bool sched_admit(const ExecView &ev, int task)
     uint32_t *run = reinterpret_cast<uint32_t *>(ev.task_running + task);
     uint32_t *occ = reinterpret_cast<uint32_t *>(&ev.st->occ);
     const uint32_t share = (uint32_t)ev.task_budget;
+    uint32_t polls = 0;
     for (;;) {
         const uint32_t r = w_load<AT>(run);
         if (r > 0 && r < (uint32_t)ev.task_cap) {
@@ -224,7 +241,7 @@ MU_HD bool sched_admit(const ExecView &ev, int task)
                 w_add<AT>(occ, (uint32_t)(-(int32_t)share));
             }
         }
-        if (sched_stopped<AT>(ev))
+        if (sched_stopped<AT>(ev, polls))
             return false;
         AT::pause();
     }

@@ -33,6 +33,15 @@ struct HostAtom {
     static bool lane0() { return true; }
     static uint32_t bcast(uint32_t v) { return v; }
     static uint32_t load(uint32_t *p) { return __atomic_load_n(p, __ATOMIC_RELAXED); }
+    static SchedPeek peek(SchedState *st)
+    {
+        SchedPeek r;
+        for (int p = 0; p < NPRIO; p++)
+            r.cnt[p] = __atomic_load_n(&st->cnt[p], __ATOMIC_RELAXED);
+        r.done = __atomic_load_n(&st->done, __ATOMIC_RELAXED);
+        r.abort = __atomic_load_n(&st->abort, __ATOMIC_RELAXED);
+        return r;
+    }
     static uint32_t load_acquire(uint32_t *p) { return __atomic_load_n(p, __ATOMIC_ACQUIRE); }
     static uint32_t load_system(uint32_t *p) { return __atomic_load_n(p, __ATOMIC_ACQUIRE); }
     static void store(uint32_t *p, uint32_t v) { __atomic_store_n(p, v, __ATOMIC_RELAXED); }

@@ -100,19 +100,30 @@ struct UnitDesc {
 };
 static_assert(sizeof(UnitDesc) == 128, "UnitDesc must stay 128 bytes");
 
-// Per-run mutable scheduler state, all in device memory.
+// Per-run mutable scheduler state, all in device memory.  The words an idle
+// worker looks at come first, in one 128-byte line that one load of a wave
+// covers; the counters that claims and producers update sit in lines of
+// their own, so the polling loads do not queue behind those atomics.
 struct SchedState {
     int32_t cnt[NPRIO];   // queued, unclaimed items per priority ring
-    uint32_t head[NPRIO]; // next ring position to hand out
-    uint32_t tail[NPRIO]; // next ring position to reserve
     uint32_t done;        // items of completed units
     uint32_t abort;       // set on a time-out or a host abort; every workgroup exits
     uint32_t err;         // 1 = no progress for the time-out, 2 = poll limit, 3 = broken DAG,
                           // 4 = aborted by the host
+    uint32_t pad0_[25];
+    uint32_t head[NPRIO]; // next ring position to hand out
+    uint32_t pad1_[28];
+    uint32_t tail[NPRIO]; // next ring position to reserve
     int32_t occ;          // CU budget of the running tasks, percent of the GPU (FLAGS_OCCUP)
-    uint32_t pad_[4];
+    uint32_t pad2_[27];
 };
-static_assert(sizeof(SchedState) == 80, "SchedState layout");
+static_assert(sizeof(SchedState) == 384, "SchedState layout");
+
+// A snapshot of the words an idle worker looks at.
+struct SchedPeek {
+    int32_t cnt[NPRIO];
+    uint32_t done, abort;
+};
 
 // Everything the device scheduler needs, passed by value to the kernels.
 struct ExecView {
