@@ -45,6 +45,14 @@ struct DevAtom {
         r.abort = (uint32_t)__builtin_amdgcn_readlane(v, 5);
         return r;
     }
+    // whether this workgroup claims now, with `cnt` items queued and `tries`
+    // polls that saw some: chance 2^(tries + 1) cnt / grid
+    static __device__ __forceinline__ bool lot(uint32_t cnt, uint32_t tries)
+    {
+        const uint32_t r = ((uint32_t)clock64() + blockIdx.x * 0x9e3779b9u) * 0x85ebca6bu;
+        return ((uint64_t)gridDim.x * (uint32_t)__builtin_amdgcn_readfirstlane(r >> 8) >> 24) <
+               ((uint64_t)cnt << (tries + 1));
+    }
     static __device__ __forceinline__ uint32_t load_acquire(uint32_t *p)
     {
         return __hip_atomic_load(p, __ATOMIC_ACQUIRE, AGENT);

@@ -161,12 +161,21 @@ MU_HD int sched_pop(const ExecView &ev, uint32_t &calls)
     uint64_t t0 = 0, idle = 0;
     uint32_t seen = 0, polls = 0;
     bool first = true;
+    uint32_t tries = 0;  // polls that saw an item since the last one that saw none
     for (;;) {
         const SchedPeek s = AT::peek(ev.st);
         if (s.abort)
             return -1;
+        bool any = false;
         for (int p = 0; p < NPRIO; p++) {
             if (s.cnt[p] <= 0)
+                continue;
+            any = true;
+            // a few items and hundreds of idle workers: about twice as many
+            // claim as there are items, twice as many on every further poll
+            // (all of them taking and giving back the count cost 50 us and
+            // more per push in the nested factorizations)
+            if (!AT::lot((uint32_t)s.cnt[p], tries))
                 continue;
             uint32_t *cnt = reinterpret_cast<uint32_t *>(&ev.st->cnt[p]);
             if ((int32_t)w_add<AT>(cnt, 0xffffffffu) <= 0) {
@@ -188,7 +197,8 @@ MU_HD int sched_pop(const ExecView &ev, uint32_t &calls)
                 AT::pause();
             }
         }
-        // nothing queued: finish, stop, or wait with the watchdog armed
+        tries = any ? (tries < 16 ? tries + 1 : 16) : 0;
+        // nothing claimed: finish, stop, or wait with the watchdog armed
         if (s.done >= ev.nitems)
             return -1;
         if ((++polls & (SCHED_HOST_POLLS - 1)) == 0 && sched_host_stopped<AT>(ev))

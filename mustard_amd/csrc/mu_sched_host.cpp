@@ -42,6 +42,7 @@ struct HostAtom {
         r.abort = __atomic_load_n(&st->abort, __ATOMIC_RELAXED);
         return r;
     }
+    static bool lot(uint32_t, uint32_t) { return true; }
     static uint32_t load_acquire(uint32_t *p) { return __atomic_load_n(p, __ATOMIC_ACQUIRE); }
     static uint32_t load_system(uint32_t *p) { return __atomic_load_n(p, __ATOMIC_ACQUIRE); }
     static void store(uint32_t *p, uint32_t v) { __atomic_store_n(p, v, __ATOMIC_RELAXED); }
