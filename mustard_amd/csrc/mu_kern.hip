@@ -27,18 +27,18 @@ __global__ MU_GEMM_KERNEL void k_batch_gemm(const UnitDesc *units, const uint32_
     run_gemm_item(d, (int)(item - d.item_base), smem);
 }
 
-// Diagonal GETRF/POTRF (and precision conversions), 4 waves held to 168
-// registers per lane: a CU running three GEMM workgroups (104 registers per
-// wave) still has room for it, so the diagonal factorization of the next step
-// starts as soon as one bulk GEMM workgroup leaves a CU instead of waiting for
-// the bulk update to drain.
-__global__ __launch_bounds__(WG_THREADS) __attribute__((amdgpu_waves_per_eu(3, 3))) void
+// Diagonal GETRF/POTRF (and precision conversions), 4 waves held to 200
+// registers per lane (the attribute counts half of the unified file): a CU
+// running three GEMM workgroups (104 registers per wave) has room for it, so
+// the diagonal factorization of the next step starts as soon as one bulk GEMM
+// workgroup leaves a CU instead of waiting for the bulk update to drain.
+__global__ __launch_bounds__(WG_THREADS) __attribute__((amdgpu_num_vgpr(100))) void
 k_batch_small(const UnitDesc *units, const uint32_t *item_unit, const uint32_t *items)
 {
     __shared__ double smem[LDS_SMALL];
     const uint32_t item = items[blockIdx.x];
     const UnitDesc d = units[item_unit[item]];
-    run_small_item<4>(d, (int)(item - d.item_base), smem);
+    run_small_item(d, (int)(item - d.item_base), smem);
 }
 
 // Reduced-precision GEMM/SYRK units whose operands are k-contiguous in

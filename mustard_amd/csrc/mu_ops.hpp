@@ -1214,32 +1214,40 @@ __device__ __forceinline__ void report_info(const UnitDesc &u, int col)
 }
 
 // ---------------------------------------------------------------------------
-// Blocked diagonal factorizations of an n x n tile (n <= SMALL_MAX), right-
-// looking over panels of 16 columns: no-pivot LU (GETRF) and lower Cholesky
-// (POTRF).  The tile sits in registers in the FP64 MFMA result layout --
-// 16 x 16 blocks, block-column j held by wave j % NW, so with 4 waves a
-// lane holds 2 block-columns x 8 blocks x 4 doubles and with 8 waves one
-// (element e of lane l of a block: row 4e + l/16, column l%16).  Panel p:
-//   * its owner wave (p % NW) copies block-column p to LDS and factors the
-//     panel alone, one lane per row (rows l and l + 64), the pivot row (LU)
-//     or the column's entries of the diagonal block (Cholesky) broadcast by
-//     readlane -- no barrier inside the panel; for LU it also forms the
-//     inverse of the unit lower 16 x 16 diagonal block;
-//   * after one barrier every wave updates its block-columns right of p on
-//     MFMA: LU forms U12 = inv(L11) A12 (four MFMAs; the result layout is
-//     the B operand of the next MFMAs) and A22 -= L21 U12; Cholesky
-//     A22 -= L21 L21^T on the lower blocks; L21 is read from the panel in
-//     LDS as the A operand;
-//   * a second barrier frees the panel buffer.
+// Blocked diagonal factorizations of an n x n tile (n <= SMALL_MAX): no-pivot
+// LU (GETRF) and lower Cholesky (POTRF), right-looking over 16 x 16 blocks on
+// four waves.  They are the serial chain of every tiled factorization, and
+// beside GEMM workgroups each of their vector instructions waits for a
+// 64-cycle FP64 MFMA, so what counts is the number of instructions in a row:
+//   * only the 16 x 16 diagonal block is factored column by column, by the
+//     wave that owns its block row, one matrix row per lane.  The pivot row /
+//     column reaches the other lanes inside the FMA itself (v_fmac_f64 with
+//     a row_newbcast operand) instead of two readlanes per element;
+//   * the same wave forms the inverse(s) of the factored block with the same
+//     instruction, so every other block of the panel is one product with a
+//     16 x 16 inverse on MFMA instead of a sweep over its rows;
+//   * the trailing update is MFMA on registers.
+// Alone, order 125: POTRF 37 -> 24 us, GETRF 91 -> 38 us against the form that
+// swept all 128 rows with readlanes and kept inv(L11) only.
+//
+// Registers: block (i, j) lives on the wave of its block row (rows w and
+// w + 4 on wave w) transposed in the MFMA result layout: element e of lane
+// (li, lk) is A(16 i + li, 16 j + 4 e + lk).  That is the B operand of A_ij^T
+// and the A operand of A_ij, and a global access covers 16 consecutive rows.
 // Rows and columns past n are the identity, so the padded factorization is
 // the n x n one; only the n x n part (Cholesky: its lower triangle) is
-// stored.  Zero pivots / non-positive minors report LAPACK-style info and
-// the factorization continues (the factors then hold inf / nan).
+// stored, each block as soon as it is final.  Zero pivots / non-positive
+// minors report LAPACK-style info and the factorization continues (the
+// factors then hold inf / nan).
 // ---------------------------------------------------------------------------
-constexpr int BF_LD = 17;                          // LDS row stride of the panel
-constexpr int LDS_SMALL_PANEL = SMALL_MAX * BF_LD;  // 128 x 16 panel (17 KB)
-// + inv(L11) for LU, + 1 / diag(L11) for Cholesky
-constexpr int LDS_SMALL_BLK = LDS_SMALL_PANEL + 16 * BF_LD + 16;
+constexpr int BF_LD = 17;                 // LDS row stride of a 16 x 16 block
+constexpr int BF_BLK = 16 * BF_LD;        // doubles of such a block
+// POTRF: the diagonal block / its inverse, two factored diagonal blocks, and
+// the solved panel in register format; GETRF: two inverses, two factored
+// diagonal blocks, the raw and the solved row panel
+constexpr int LDS_POTRF = 3 * BF_BLK + 8 * 256;
+constexpr int LDS_GETRF = 4 * BF_BLK + 7 * BF_BLK + 7 * 256;
+constexpr int LDS_SMALL_BLK = LDS_GETRF > LDS_POTRF ? LDS_GETRF : LDS_POTRF;
 
 // 1/x and 1/sqrt(x) in FP64 from the hardware estimates (v_rcp_f64,
 // v_rsq_f64) and two Newton steps each (r <- r + r (1 - x r), r <- r + r
@@ -1262,234 +1270,628 @@ __device__ __forceinline__ double rsq_nr(double x)
     return fma(r, fma(-h * r, r, 0.5), r);
 }
 
-__device__ __forceinline__ double readlane_d(double v, int lane)
+// Lane L's v of every group of 16 lanes.
+template <int L>
+__device__ __forceinline__ double bcast16(double v)
 {
     const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffll), lane);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), 0x150 + L, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x150 + L, 0xf, 0xf, false);
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-template <bool CHOL, int NW = 4>
-__device__ __attribute__((always_inline)) inline void factor_small_blk(const UnitDesc &u,
-                                                                       double *smem)
+// d[k] -= (s of lane k of the group) * m for k = K .. 15.  A DPP operand may
+// be read two wait states after a VALU write of it; the s_nop (8 cycles) at
+// the head of each asm block covers whatever the compiler put before it, so
+// the blocks are as wide as asm operands allow.
+#define MU_FMAC(i, src, l)                                                                     \
+    "v_fmac_f64_dpp %[d" #i "], " #src ", -%[m] row_newbcast:%[" #l "] row_mask:0xf bank_mask:0xf\n\t"
+#define MU_IO(i) [d##i] "+&v"(d[K + i])
+#define MU_L(i) [l##i] "n"(K + i)
+template <int K>
+__device__ __forceinline__ void fms_lane(double (&d)[16], double s, double m)
 {
-    // NW waves (4 or 8); block-column j is held by wave j % NW
-    static_assert(NW == 4 || NW == 8, "4 or 8 waves");
-    constexpr int JJ = 8 / NW;
-    const int n = u.m, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int q = lane >> 4, cl = lane & 15;
-    const int nb = (n + 15) >> 4;
-    MU_G double *a = gp(u.c);
-    const size_t lda = u.ldc;
-    double *P = smem;                     // panel: row r (0..127), column c at P[r * 17 + c]
-    double *Li = smem + LDS_SMALL_PANEL;  // LU: inv(L11), row-major, stride 17
-    double *Rc = Li + 16 * BF_LD;         // Cholesky: 1 / diag(L11) of the panel
-    // the diagonal factorization is the serial chain of the whole DAG: its
-    // waves issue ahead of the GEMM waves sharing their SIMDs
-    __builtin_amdgcn_s_setprio(3);
-
-    v4d R[JJ][8];  // block (i, w + NW jj)
-#pragma unroll
-    for (int jj = 0; jj < JJ; jj++)
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int r = 16 * i + 4 * e + q, c = 16 * (w + NW * jj) + cl;
-                double v = r == c ? 1.0 : 0.0;
-                if (r < n && c < n && (!CHOL || r >= c))
-                    v = a[r + (size_t)c * lda];
-                R[jj][i][e] = v;
-            }
-
-    for (int p = 0; p < nb; p++) {
-        const int jp = p / NW;  // the owner's register column of block-column p
-        if (w == p % NW) {
-            // ---- panel: block-column p, rows 16p .. 127, to LDS ----
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-                if (i >= p) {
-                    const v4d blk = (JJ > 1 && jp) ? R[JJ - 1][i] : R[0][i];
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        P[(16 * i + 4 * e + q) * BF_LD + cl] = blk[e];
-                }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            const int p0 = 16 * p;
-            // sweep 1: rows p0 .. p0 + 63, lane l on row p0 + l; the pivot
-            // row of column c is lane c's
-            {
-                const int r = p0 + lane;
-                const bool in = r < SMALL_MAX;
-                // lanes past the tile read the last row (their results are
-                // dropped): no branch around the loads
-                const double *src = P + (in ? r : SMALL_MAX - 1) * BF_LD;
-                double x[16];
-#pragma unroll
-                for (int c = 0; c < 16; c++)
-                    x[c] = src[c];
-                // the first failing column of the panel, uniform; reported
-                // once after the sweep instead of a branch in every column
-                int bad = 16;
-#pragma unroll
-                for (int c = 0; c < 16; c++) {
-                    const double piv = readlane_d(x[c], c);
-                    if (!CHOL) {
-                        bad = min(bad, piv == 0.0 ? c : 16);
-                        const double l = lane > c ? x[c] * rcp_nr(piv) : 0.0;
-                        if (lane > c)
-                            x[c] = l;
-                        // lane c's own row keeps its values (multiplier 0)
-#pragma unroll
-                        for (int k = c + 1; k < 16; k++)
-                            x[k] = fma(-l, readlane_d(x[k], c), x[k]);
-                    } else {
-                        bad = min(bad, piv > 0.0 ? 16 : c);
-                        const double rd = rsq_nr(piv);
-                        Rc[c] = rd;
-                        // every lane, no masks: lane c gets piv * rd, the
-                        // lanes above it only change the diagonal block's
-                        // upper part, which nothing reads
-                        x[c] *= rd;
-#pragma unroll
-                        for (int k = c + 1; k < 16; k++)  // L[p0 + k][c] is lane k's
-                            x[k] = fma(-x[c], readlane_d(x[c], k), x[k]);
-                    }
-                }
-                if (bad < 16 && lane == 0)
-                    report_info(u, p0 + bad);
-#pragma unroll
-                for (int c = 0; c < 16; c++)
-                    if (in)
-                        P[r * BF_LD + c] = x[c];
-            }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            // sweep 2: rows p0 + 64 .. 127 against the finished diagonal
-            // block in LDS (LU: L21 = A21 inv(U11); Cholesky: A21 inv(L11^T))
-            if (p0 + 64 < SMALL_MAX) {
-                const int r = p0 + 64 + lane;
-                const bool in = r < SMALL_MAX;
-                const double *src = P + (in ? r : SMALL_MAX - 1) * BF_LD;
-                double y[16];
-#pragma unroll
-                for (int c = 0; c < 16; c++)
-                    y[c] = src[c];
-#pragma unroll
-                for (int c = 0; c < 16; c++) {
-                    const double *dr = P + (p0 + c) * BF_LD;  // LU: row c of U11
-                    if (!CHOL) {
-                        y[c] *= rcp_nr(dr[c]);  // the multiplier of sweep 1's rows
-#pragma unroll
-                        for (int k = c + 1; k < 16; k++)
-                            y[k] = fma(-y[c], dr[k], y[k]);
-                    } else {
-                        y[c] *= Rc[c];  // 1 / L11[c][c], as sweep 1 scaled its rows
-#pragma unroll
-                        for (int k = c + 1; k < 16; k++)  // L11[k][c]
-                            y[k] = fma(-y[c], P[(p0 + k) * BF_LD + c], y[k]);
-                    }
-                }
-#pragma unroll
-                for (int c = 0; c < 16; c++)
-                    if (in)
-                        P[r * BF_LD + c] = y[c];
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            }
-            if (!CHOL && lane < 16) {
-                // column `lane` of inv(L11) (unit lower): forward substitution
-                double z[16];
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    double s = r == lane ? 1.0 : 0.0;
-#pragma unroll
-                    for (int k = 0; k < r; k++)
-                        s = fma(-P[(p0 + r) * BF_LD + k], z[k], s);
-                    z[r] = s;
-                }
-#pragma unroll
-                for (int r = 0; r < 16; r++)
-                    Li[r * BF_LD + lane] = z[r];
-            }
-            // the factored panel back into the owner's registers
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-                if (i >= p) {
-                    v4d blk;
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        blk[e] = P[(16 * i + 4 * e + q) * BF_LD + cl];
-                    if (CHOL && i == p)  // keep the diagonal block's upper part as loaded
-#pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            if (4 * e + q < cl)
-                                blk[e] = 0.0;
-                    if (JJ > 1 && jp)
-                        R[JJ - 1][i] = blk;
-                    else
-                        R[0][i] = blk;
-                }
-        }
-        lds_barrier();
-        // ---- trailing update of this wave's block-columns j > p ----
-#pragma unroll
-        for (int jj = 0; jj < JJ; jj++) {
-            const int j = w + NW * jj;
-            if (j <= p || j >= nb)
-                continue;
-            if (!CHOL) {
-                // U12 = inv(L11) A12, block (p, j)
-                v4d up = R[jj][0];
-#pragma unroll
-                for (int i = 1; i < 8; i++)
-                    if (i == p)
-                        up = R[jj][i];
-                v4d acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-                for (int kk = 0; kk < 4; kk++)
-                    acc = mfma_f64(Li[cl * BF_LD + 4 * kk + q], up[kk], acc);
-#pragma unroll
-                for (int i = 0; i < 8; i++)
-                    if (i == p)
-                        R[jj][i] = acc;
-#pragma unroll
-                for (int i = 0; i < 8; i++)
-                    if (i > p && i < nb) {
-                        v4d c4 = R[jj][i];
-#pragma unroll
-                        for (int kk = 0; kk < 4; kk++)
-                            c4 = mfma_f64(-P[(16 * i + cl) * BF_LD + 4 * kk + q], acc[kk], c4);
-                        R[jj][i] = c4;
-                    }
-            } else {
-                double bj[4];
-#pragma unroll
-                for (int kk = 0; kk < 4; kk++)
-                    bj[kk] = P[(16 * j + cl) * BF_LD + 4 * kk + q];
-#pragma unroll
-                for (int i = 0; i < 8; i++)
-                    if (i >= j && i < nb) {
-                        v4d c4 = R[jj][i];
-#pragma unroll
-                        for (int kk = 0; kk < 4; kk++)
-                            c4 = mfma_f64(-P[(16 * i + cl) * BF_LD + 4 * kk + q], bj[kk], c4);
-                        R[jj][i] = c4;
-                    }
-            }
-        }
-        lds_barrier();
+    if constexpr (K <= 4) {
+        asm("s_nop 1\n\t" MU_FMAC(0, %[s], l0) MU_FMAC(1, %[s], l1) MU_FMAC(2, %[s], l2) MU_FMAC(3, %[s], l3) MU_FMAC(4, %[s], l4) MU_FMAC(5, %[s], l5) MU_FMAC(6, %[s], l6) MU_FMAC(7, %[s], l7) MU_FMAC(8, %[s], l8) MU_FMAC(9, %[s], l9) MU_FMAC(10, %[s], l10) MU_FMAC(11, %[s], l11)
+            : MU_IO(0), MU_IO(1), MU_IO(2), MU_IO(3), MU_IO(4), MU_IO(5), MU_IO(6), MU_IO(7), MU_IO(8), MU_IO(9), MU_IO(10), MU_IO(11)
+            : [s] "v"(s), [m] "v"(m), MU_L(0), MU_L(1), MU_L(2), MU_L(3), MU_L(4), MU_L(5), MU_L(6), MU_L(7), MU_L(8), MU_L(9), MU_L(10), MU_L(11));
+        fms_lane<K + 12>(d, s, m);
+    } else if constexpr (K <= 8) {
+        asm("s_nop 1\n\t" MU_FMAC(0, %[s], l0) MU_FMAC(1, %[s], l1) MU_FMAC(2, %[s], l2) MU_FMAC(3, %[s], l3) MU_FMAC(4, %[s], l4) MU_FMAC(5, %[s], l5) MU_FMAC(6, %[s], l6) MU_FMAC(7, %[s], l7)
+            : MU_IO(0), MU_IO(1), MU_IO(2), MU_IO(3), MU_IO(4), MU_IO(5), MU_IO(6), MU_IO(7)
+            : [s] "v"(s), [m] "v"(m), MU_L(0), MU_L(1), MU_L(2), MU_L(3), MU_L(4), MU_L(5), MU_L(6), MU_L(7));
+        fms_lane<K + 8>(d, s, m);
+    } else if constexpr (K <= 10) {
+        asm("s_nop 1\n\t" MU_FMAC(0, %[s], l0) MU_FMAC(1, %[s], l1) MU_FMAC(2, %[s], l2) MU_FMAC(3, %[s], l3) MU_FMAC(4, %[s], l4) MU_FMAC(5, %[s], l5)
+            : MU_IO(0), MU_IO(1), MU_IO(2), MU_IO(3), MU_IO(4), MU_IO(5)
+            : [s] "v"(s), [m] "v"(m), MU_L(0), MU_L(1), MU_L(2), MU_L(3), MU_L(4), MU_L(5));
+        fms_lane<K + 6>(d, s, m);
+    } else if constexpr (K <= 12) {
+        asm("s_nop 1\n\t" MU_FMAC(0, %[s], l0) MU_FMAC(1, %[s], l1) MU_FMAC(2, %[s], l2) MU_FMAC(3, %[s], l3)
+            : MU_IO(0), MU_IO(1), MU_IO(2), MU_IO(3)
+            : [s] "v"(s), [m] "v"(m), MU_L(0), MU_L(1), MU_L(2), MU_L(3));
+        fms_lane<K + 4>(d, s, m);
+    } else if constexpr (K <= 13) {
+        asm("s_nop 1\n\t" MU_FMAC(0, %[s], l0) MU_FMAC(1, %[s], l1) MU_FMAC(2, %[s], l2)
+            : MU_IO(0), MU_IO(1), MU_IO(2)
+            : [s] "v"(s), [m] "v"(m), MU_L(0), MU_L(1), MU_L(2));
+        fms_lane<K + 3>(d, s, m);
+    } else if constexpr (K <= 14) {
+        asm("s_nop 1\n\t" MU_FMAC(0, %[s], l0) MU_FMAC(1, %[s], l1)
+            : MU_IO(0), MU_IO(1)
+            : [s] "v"(s), [m] "v"(m), MU_L(0), MU_L(1));
+        fms_lane<K + 2>(d, s, m);
+    } else if constexpr (K <= 15) {
+        asm("s_nop 1\n\t" MU_FMAC(0, %[s], l0)
+            : MU_IO(0)
+            : [s] "v"(s), [m] "v"(m), MU_L(0));
+        fms_lane<K + 1>(d, s, m);
     }
+}
+// d[k] -= (d[k] of lane L) * m for k = K .. 15
+template <int L, int K>
+__device__ __forceinline__ void fms_self(double (&d)[16], double m)
+{
+    if constexpr (K <= 4) {
+        asm("s_nop 1\n\t" MU_FMAC(0, %[d0], l) MU_FMAC(1, %[d1], l) MU_FMAC(2, %[d2], l) MU_FMAC(3, %[d3], l) MU_FMAC(4, %[d4], l) MU_FMAC(5, %[d5], l) MU_FMAC(6, %[d6], l) MU_FMAC(7, %[d7], l) MU_FMAC(8, %[d8], l) MU_FMAC(9, %[d9], l) MU_FMAC(10, %[d10], l) MU_FMAC(11, %[d11], l)
+            : MU_IO(0), MU_IO(1), MU_IO(2), MU_IO(3), MU_IO(4), MU_IO(5), MU_IO(6), MU_IO(7), MU_IO(8), MU_IO(9), MU_IO(10), MU_IO(11)
+            : [m] "v"(m), [l] "n"(L));
+        fms_self<L, K + 12>(d, m);
+    } else if constexpr (K <= 8) {
+        asm("s_nop 1\n\t" MU_FMAC(0, %[d0], l) MU_FMAC(1, %[d1], l) MU_FMAC(2, %[d2], l) MU_FMAC(3, %[d3], l) MU_FMAC(4, %[d4], l) MU_FMAC(5, %[d5], l) MU_FMAC(6, %[d6], l) MU_FMAC(7, %[d7], l)
+            : MU_IO(0), MU_IO(1), MU_IO(2), MU_IO(3), MU_IO(4), MU_IO(5), MU_IO(6), MU_IO(7)
+            : [m] "v"(m), [l] "n"(L));
+        fms_self<L, K + 8>(d, m);
+    } else if constexpr (K <= 10) {
+        asm("s_nop 1\n\t" MU_FMAC(0, %[d0], l) MU_FMAC(1, %[d1], l) MU_FMAC(2, %[d2], l) MU_FMAC(3, %[d3], l) MU_FMAC(4, %[d4], l) MU_FMAC(5, %[d5], l)
+            : MU_IO(0), MU_IO(1), MU_IO(2), MU_IO(3), MU_IO(4), MU_IO(5)
+            : [m] "v"(m), [l] "n"(L));
+        fms_self<L, K + 6>(d, m);
+    } else if constexpr (K <= 12) {
+        asm("s_nop 1\n\t" MU_FMAC(0, %[d0], l) MU_FMAC(1, %[d1], l) MU_FMAC(2, %[d2], l) MU_FMAC(3, %[d3], l)
+            : MU_IO(0), MU_IO(1), MU_IO(2), MU_IO(3)
+            : [m] "v"(m), [l] "n"(L));
+        fms_self<L, K + 4>(d, m);
+    } else if constexpr (K <= 13) {
+        asm("s_nop 1\n\t" MU_FMAC(0, %[d0], l) MU_FMAC(1, %[d1], l) MU_FMAC(2, %[d2], l)
+            : MU_IO(0), MU_IO(1), MU_IO(2)
+            : [m] "v"(m), [l] "n"(L));
+        fms_self<L, K + 3>(d, m);
+    } else if constexpr (K <= 14) {
+        asm("s_nop 1\n\t" MU_FMAC(0, %[d0], l) MU_FMAC(1, %[d1], l)
+            : MU_IO(0), MU_IO(1)
+            : [m] "v"(m), [l] "n"(L));
+        fms_self<L, K + 2>(d, m);
+    } else if constexpr (K <= 15) {
+        asm("s_nop 1\n\t" MU_FMAC(0, %[d0], l)
+            : MU_IO(0)
+            : [m] "v"(m), [l] "n"(L));
+        fms_self<L, K + 1>(d, m);
+    }
+}
+#undef MU_FMAC
+#undef MU_IO
+#undef MU_L
 
+// The head of column C: d[C + 1 .. C + 3] updated (SELF: with their own lane
+// C, as fms_self<C>; else with s of lanes C + 1 .. C + 3, as fms_lane).  The
+// block ends two wait states after the write of d[C + 1], which a DPP move
+// (the next pivot's broadcast) may then read.
+#define MU_F3(s0, s1, s2, l0, l1, l2)                                                         \
+    "s_nop 1\n\tv_fmac_f64_dpp %0, " s0 ", -%4 row_newbcast:" l0 " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f64_dpp %1, " s1 ", -%4 row_newbcast:" l1 " row_mask:0xf bank_mask:0xf\n\t"        \
+    "v_fmac_f64_dpp %2, " s2 ", -%4 row_newbcast:" l2 " row_mask:0xf bank_mask:0xf"
+template <bool SELF, int C>
+__device__ __forceinline__ void col_head(double (&d)[16], double s, double m)
+{
+    if constexpr (C < 13) {
+        if constexpr (SELF)
+            asm(MU_F3("%0", "%1", "%2", "%5", "%5", "%5")
+                : "+&v"(d[C + 1]), "+&v"(d[C + 2]), "+&v"(d[C + 3])
+                : "v"(s), "v"(m), "n"(C));
+        else
+            asm(MU_F3("%3", "%3", "%3", "%5", "%6", "%7")
+                : "+&v"(d[C + 1]), "+&v"(d[C + 2]), "+&v"(d[C + 3])
+                : "v"(s), "v"(m), "n"(C + 1), "n"(C + 2), "n"(C + 3));
+    } else if constexpr (C < 15) {
+        if constexpr (SELF)
+            fms_self<C, C + 1>(d, m);
+        else
+            fms_lane<C + 1>(d, s, m);
+        asm("s_nop 1" : "+v"(d[C + 1]));
+    }
+}
+#undef MU_F3
+
+// Cholesky of a 16 x 16 block, lane li holding row li in x (lower part
+// valid; every group of 16 lanes the same block), and column li of inv(L) in
+// z (the identity's on entry), row C of it stored to W once final.  `piv` is
+// the pivot of column C, `bad` the first failing column.
+template <int C>
+__device__ __forceinline__ void potrf16(double (&x)[16], double (&z)[16], double *W, double piv,
+                                        int &bad)
+{
+    if constexpr (C < 16) {
+        bad = min(bad, piv > 0.0 ? 16 : C);
+        const double rd = rsq_nr(piv);
+        x[C] *= rd;
+        if constexpr (C < 15) {
+            col_head<false, C>(x, x[C], x[C]);
+            piv = bcast16<C + 1>(x[C + 1]);
+        }
+        z[C] *= rd;
+        W[C * BF_LD] = z[C];
+        if constexpr (C < 13)
+            fms_lane<C + 4>(x, x[C], x[C]);
+        fms_lane<C + 1>(z, x[C], z[C]);
+        potrf16<C + 1>(x, z, W, piv, bad);
+    }
+}
+
+// No-pivot elimination of a 16 x 16 block, lane li holding row li in x:
+// afterwards x[c] is the multiplier for c < li (unit lower factor) and the
+// upper factor's row otherwise; z as above for the unit lower factor, row C
+// stored to W scaled by 1 / pivot in the lanes with `scale`.
+template <int C>
+__device__ __forceinline__ void getrf16(double (&x)[16], double (&z)[16], double *W, double piv,
+                                        int li, bool scale, int &bad)
+{
+    if constexpr (C < 16) {
+        bad = min(bad, piv == 0.0 ? C : 16);
+        const double rd = rcp_nr(piv);
+        const double m = li > C ? x[C] * rd : 0.0;
+        x[C] = li > C ? m : x[C];
+        if constexpr (C < 15) {
+            col_head<true, C>(x, m, m);
+            piv = bcast16<C + 1>(x[C + 1]);
+        }
+        W[C * BF_LD] = scale ? z[C] * rd : z[C];
+        if constexpr (C < 13)
+            fms_self<C, C + 4>(x, m);
+        fms_lane<C + 1>(z, m, z[C]);
+        getrf16<C + 1>(x, z, W, piv, li, scale, bad);
+    }
+}
+
+// this wave's own LDS traffic is done (no barrier)
+__device__ __forceinline__ void lds_wait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// Block (i, j) of an n x n tile into its register format; rows and columns
+// past n read the last one.  The scheduling barrier keeps one block's
+// addresses from living beside the next one's.
+__device__ __forceinline__ void load_blk16(v4d &v, const MU_G double *a, unsigned lda, int n, int i,
+                                           int j, int li, int lk)
+{
+    const unsigned r = min(16 * i + li, n - 1);
 #pragma unroll
-    for (int jj = 0; jj < JJ; jj++)
+    for (int e = 0; e < 4; e++)
+        v[e] = a[r + (unsigned)min(16 * j + 4 * e + lk, n - 1) * lda];
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// acc[] -= the products of k-steps e = 0 .. 3, a block at a time: MFMA A
+// operands from LDS (register format, blocks 256 apart), the next block's
+// read ahead of this block's MFMAs.
+template <int J0, int J1>
+__device__ __forceinline__ void update_row(v4d *acc, const double *lds, const v4d &x)
+{
+    double f[2][4];
 #pragma unroll
-        for (int i = 0; i < 8; i++)
+    for (int e = 0; e < 4; e++)
+        f[J0 & 1][e] = lds[J0 * 256 + e * 64];
+#pragma unroll
+    for (int j = J0; j < J1; j++) {
+        if (j + 1 < J1)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                f[(j + 1) & 1][e] = lds[(j + 1) * 256 + e * 64];
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            acc[j] = mfma_f64(f[j & 1][e], x[e], acc[j]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+struct SmallCtx {
+    int n, nb, w, li, lk, lane;
+    MU_G double *a;
+    unsigned lda;  // uniform (a scalar register)
+    // Once per step: hides that lane and leading dimension are the same in
+    // every step.  Otherwise the addresses of all eight steps' loads and
+    // stores are computed ahead of the loop and live (spilled) across it.
+    __device__ __forceinline__ void refresh()
+    {
+        asm volatile("" : "+v"(lane), "+s"(lda));
+        li = lane & 15;
+        lk = lane >> 4;
+    }
+};
+
+// Block (i, P) of the factor from its register format.
+template <int P>
+__device__ __forceinline__ void store_blk16(const SmallCtx &c, int i, const v4d &x)
+{
+    if (16 * i + c.li < c.n)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            (c.a + 16 * i + (size_t)(16 * P + 4 * e) * c.lda)[c.li + c.lk * c.lda] = x[e];
+}
+
+// The owner of block row p + 1 hands its diagonal block to the factoring wave.
+__device__ __forceinline__ void put_diag16(const SmallCtx &c, double *W, const v4d &D)
+{
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        W[c.li * BF_LD + 4 * e + c.lk] = D[e];
+}
+
+// Waves.  Four waves, block rows w and w + 4 on wave w.  Wave 0 also factors
+// every diagonal block: its row 0 only goes through LDS, so that it holds one
+// block row beside the 64 registers of the block's columns.  At 200 registers
+// per lane the kernel starts on a CU as soon as one of four GEMM workgroups
+// (104 each) leaves it; at 256 it had to find two gone and waited 400 us and
+// more per node beside a bulk update.  Barriers per step: the inverse is in
+// LDS (A), the solved panel is in LDS (B), the next diagonal block is in LDS
+// (C).  The trailing update of the other blocks runs beside the next diagonal
+// block's columns.
+//
+// The factored diagonal block p from LDS to the matrix (LOWER: its lower part).
+template <bool LOWER>
+__device__ __forceinline__ void store_diag16(const SmallCtx &c, int p, const double *D)
+{
+    if (16 * p + c.li < c.n)
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int k = 4 * e + c.lk;
+            if (LOWER ? k <= c.li : 16 * p + k < c.n)
+                (c.a + 16 * p + (size_t)(16 * p + 4 * e) * c.lda)[c.li + c.lk * c.lda] =
+                    D[c.li * BF_LD + k];
+        }
+}
+
+// Lower Cholesky.  Factoring step p: A_pp = L_pp L_pp^T, inv(L_pp) to W, L_pp
+// to D (two buffers in turn: a tile wave stores it a step later).
+__device__ __forceinline__ void potrf_diag(const SmallCtx &c, const UnitDesc &u, int p, double *W,
+                                           double *D)
+{
+    const int li = c.li;
+    double x[16], z[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+        x[k] = W[li * BF_LD + k];
+        z[k] = k == li ? 1.0 : 0.0;
+    }
+    lds_wait();
+    int bad = 16;
+    potrf16<0>(x, z, W + li, bcast16<0>(x[0]), bad);
+    if (bad < 16 && c.lane == 0)
+        report_info(u, 16 * p + bad);
+#pragma unroll
+    for (int k = 0; k < 16; k++)
+        D[li * BF_LD + k] = x[k];
+}
+
+// Tile waves, step P: L_ip^T = inv(L_pp) A_ip^T for the blocks below, stored
+// and handed on as -L_ip (Lb); then A_ij^T += (-L_jp) L_ip^T, the next
+// diagonal block first.  R0: row w, columns 0 .. 3; R1: row w + 4 (blocks
+// right of the diagonal hold nothing that is read).
+template <int P, bool W0>
+__device__ __forceinline__ void potrf_step(const SmallCtx &c, v4d (&R0)[4], v4d (&R1)[8],
+                                           double *W, double *Lb)
+{
+    const bool on0 = !W0 && P < 3 && c.w > P && c.w < c.nb;
+    const bool on1 = c.w + 4 > P && c.w + 4 < c.nb;
+    v4d X0 = {0.0, 0.0, 0.0, 0.0}, X1 = X0;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {  // a finished row solves a block nothing reads
+        const double wv = W[c.li * BF_LD + 4 * e + c.lk];
+        if constexpr (!W0 && P < 3)
+            X0 = mfma_f64(wv, R0[P][e], X0);
+        X1 = mfma_f64(wv, R1[P][e], X1);
+    }
+    auto put = [&](int i, const v4d &x) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            Lb[i * 256 + e * 64 + c.lane] = -x[e];
+    };
+    if (on0)
+        put(c.w, X0);
+    if (on1)
+        put(c.w + 4, X1);
+    lds_barrier();  // B
+    const double *L = Lb + c.lane;
+    constexpr int Q = P + 1;  // the next diagonal block
+    if (c.w == (Q & 3)) {
+        if constexpr (Q >= 4) {
+            update_row<Q, Q + 1>(R1, L, X1);
+            put_diag16(c, W, R1[Q]);
+        } else if constexpr (!W0) {
+            update_row<Q, Q + 1>(R0, L, X0);
+            put_diag16(c, W, R0[Q]);
+        }
+    }
+    lds_barrier();  // C
+    if (on0)
+        store_blk16<P>(c, c.w, X0);
+    if (on1)
+        store_blk16<P>(c, c.w + 4, X1);
+    if constexpr (!W0 && Q < 3)
+        if (on0 && c.w > Q)  // columns past w are not used
+            update_row<Q, 4>(R0, L, X0);
+    if (on1 && c.w + 4 > Q) {
+        if constexpr (!W0 || Q < 5)
+            update_row<Q, (Q < 5 ? 5 : Q + 1)>(R1, L, X1);
+        if constexpr (!W0 && Q < 5)
+            update_row<5, 6>(R1, L, X1);
+        if constexpr (!W0 && Q < 6)
+            if (c.w >= 2)
+                update_row<6, 7>(R1, L, X1);
+        if constexpr (!W0 && Q < 7)
+            if (c.w >= 3)
+                update_row<7, 8>(R1, L, X1);
+    }
+}
+
+// Step p (a switch: the register arrays need constant indices).
+template <bool W0>
+__device__ __forceinline__ void potrf_steps(const SmallCtx &c, int p, v4d (&R0)[4], v4d (&R1)[8],
+                                            double *W, double *Lb)
+{
+    switch (p) {
+    case 0: potrf_step<0, W0>(c, R0, R1, W, Lb); break;
+    case 1: potrf_step<1, W0>(c, R0, R1, W, Lb); break;
+    case 2: potrf_step<2, W0>(c, R0, R1, W, Lb); break;
+    case 3: potrf_step<3, W0>(c, R0, R1, W, Lb); break;
+    case 4: potrf_step<4, W0>(c, R0, R1, W, Lb); break;
+    case 5: potrf_step<5, W0>(c, R0, R1, W, Lb); break;
+    default: potrf_step<6, W0>(c, R0, R1, W, Lb); break;
+    }
+}
+
+template <bool W0>
+__device__ __forceinline__ void potrf_waves(SmallCtx c, const UnitDesc &u, double *W, double *D,
+                                            double *Lb)
+{
+    const int n = c.n, nb = c.nb, w = c.w, li = c.li, lk = c.lk;
+    // every load first, from addresses clamped into the tile; then the parts
+    // outside the tile and above the diagonal (uniform tests: edge blocks only)
+    v4d R0[4], R1[8];
+#pragma unroll
+    for (int j = 0; j < (W0 ? 1 : 4); j++)
+        load_blk16(R0[j], c.a, c.lda, n, w, min(j, w), li, lk);
+#pragma unroll
+    for (int j = 0; j < (W0 ? 5 : 8); j++)
+        load_blk16(R1[j], c.a, c.lda, n, w + 4, min(j, w + 4), li, lk);
+    auto mask = [&](v4d &v, int i, int j) {
+        if (i == j || i >= nb - 1)
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const int r = 16 * i + 4 * e + q, c = 16 * (w + NW * jj) + cl;
-                if (r < n && c < n && (!CHOL || r >= c))
-                    a[r + (size_t)c * lda] = R[jj][i][e];
+                const int r = 16 * i + li, k = 16 * j + 4 * e + lk;
+                v[e] = (r < n && k <= r) ? v[e] : (r == k ? 1.0 : 0.0);
             }
+    };
+#pragma unroll
+    for (int j = 0; j < (W0 ? 1 : 4); j++)
+        mask(R0[j], w, j);
+    if (W0)
+        put_diag16(c, W, R0[0]);
+#pragma unroll
+    for (int j = 0; j < (W0 ? 5 : 8); j++)
+        mask(R1[j], w + 4, j);
+    lds_barrier();  // C
+    for (int p = 0;; p++) {
+        c.refresh();
+        if (W0)
+            potrf_diag(c, u, p, W, D + (p & 1) * BF_BLK);
+        lds_barrier();  // A
+        if (p + 1 < nb)
+            potrf_steps<W0>(c, p, R0, R1, W, Lb);
+        if (w == (p & 3))
+            store_diag16<true>(c, p, D + (p & 1) * BF_BLK);
+        if (p + 1 == nb)
+            break;
+    }
+}
+
+__device__ __attribute__((always_inline)) inline void potrf_small(const UnitDesc &u, double *smem)
+{
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const SmallCtx c = {u.m,       (u.m + 15) >> 4, w, lane & 15, lane >> 4, lane, gp(u.c),
+                        (unsigned)__builtin_amdgcn_readfirstlane(u.ldc)};
+    double *W = smem, *D = W + BF_BLK, *Lb = D + 2 * BF_BLK;
+    __builtin_amdgcn_s_setprio(3);
+    if (w == 0)
+        potrf_waves<true>(c, u, W, D, Lb);
+    else
+        potrf_waves<false>(c, u, W, D, Lb);
+    __builtin_amdgcn_s_setprio(0);
+}
+
+// No-pivot LU.  Factoring step p: two groups of 16 lanes eliminate A_pp at
+// once, one on the block and one on its transpose, whose unit lower factor is
+// the transposed unit upper factor of A_pp = L D U', and invert both:
+// W1 = inv(L), W2 = inv(U)^T = D^-1 inv(U')^T.  The packed factors go to D.
+__device__ __forceinline__ void getrf_diag(const SmallCtx &c, const UnitDesc &u, int p, double *W1,
+                                           double *W2, double *D)
+{
+    const int li = c.li;
+    // groups 0 and 2: rows of the block, groups 1 and 3: its columns
+    const int g = c.lk & 1;
+    double x[16], z[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+        x[k] = W1[g ? k * BF_LD + li : li * BF_LD + k];
+        z[k] = k == li ? 1.0 : 0.0;
+    }
+    lds_wait();
+    int bad = 16;
+    getrf16<0>(x, z, (g ? W2 : W1) + li, bcast16<0>(x[0]), li, g != 0, bad);
+    if (bad < 16 && c.lane == 0)
+        report_info(u, 16 * p + bad);
+    if (g == 0)
+#pragma unroll
+        for (int k = 0; k < 16; k++)
+            D[li * BF_LD + k] = x[k];
+}
+
+// Blocks J0 .. 7 of row panel row to LDS, block j at raw + (j - 1) BF_BLK.
+template <int J0>
+__device__ __forceinline__ void put_raw16(const SmallCtx &c, const v4d (&R)[8], double *raw)
+{
+#pragma unroll
+    for (int j = J0; j < 8; j++)
+        if (j < c.nb)
+            put_diag16(c, raw + (j - 1) * BF_BLK, R[j]);
+}
+
+// Tile waves, step P: L_ip^T = inv(U)^T A_ip^T for the blocks below, a share
+// of the row panel, U_pj = inv(L) A_pj (copied to LDS raw by its owner),
+// handed on as -U_pj (Ub); then A_ij^T += (-U_pj)^T L_ip^T, the next diagonal
+// block first.  R0, R1: block rows w and w + 4.
+template <int P, bool W0>
+__device__ __forceinline__ void getrf_step(const SmallCtx &c, v4d (&R0)[8], v4d (&R1)[8],
+                                           double *W1, const double *W2, double *raw, double *Ub)
+{
+    const bool on0 = !W0 && P < 3 && c.w > P && c.w < c.nb;
+    const bool on1 = c.w + 4 > P && c.w + 4 < c.nb;
+    v4d X0 = {0.0, 0.0, 0.0, 0.0}, X1 = X0;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {  // a finished row solves a block nothing reads
+        const double wv = W2[c.li * BF_LD + 4 * e + c.lk];
+        if constexpr (!W0 && P < 3)
+            X0 = mfma_f64(wv, R0[P][e], X0);
+        X1 = mfma_f64(wv, R1[P][e], X1);
+    }
+    for (int j = P + 1 + c.w; j < c.nb; j += 4) {
+        const double *b = raw + (j - 1) * BF_BLK;
+        v4d x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            x = mfma_f64(W1[c.li * BF_LD + 4 * e + c.lk], b[(4 * e + c.lk) * BF_LD + c.li], x);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            Ub[(j - 1) * 256 + e * 64 + c.lane] = -x[e];
+            if (16 * j + c.li < c.n)
+                (c.a + 16 * P + 4 * e + (size_t)(16 * j) * c.lda)[c.lk + c.li * c.lda] = x[e];
+        }
+    }
+    lds_barrier();  // B
+    const double *U = Ub + c.lane - 256;
+    constexpr int Q = P + 1;  // the next diagonal block
+    const bool own = c.w == (Q & 3);
+    if (own) {
+        if constexpr (Q >= 4) {
+            update_row<Q, Q + 1>(R1, U, X1);
+            put_diag16(c, W1, R1[Q]);
+        } else if constexpr (!W0) {
+            update_row<Q, Q + 1>(R0, U, X0);
+            put_diag16(c, W1, R0[Q]);
+        }
+    }
+    lds_barrier();  // C
+    // columns past nb hold nothing that is read
+    if constexpr (Q < 4) {
+        if constexpr (!W0) {
+            if (own) {
+                update_row<Q + 1, 8>(R0, U, X0);
+                put_raw16<Q + 1>(c, R0, raw);
+            } else if (on0) {
+                update_row<Q, 8>(R0, U, X0);
+            }
+            if (on0)
+                store_blk16<P>(c, c.w, X0);
+        }
+        if (on1)
+            update_row<Q, 8>(R1, U, X1);
+    } else if constexpr (!W0 || Q == 4) {
+        if (own) {
+            if constexpr (Q < 7)
+                update_row<Q + 1, 8>(R1, U, X1);
+            put_raw16<Q + 1>(c, R1, raw);
+        } else if (on1) {
+            update_row<Q, 8>(R1, U, X1);
+        }
+    }
+    if (on1)
+        store_blk16<P>(c, c.w + 4, X1);
+}
+
+template <bool W0>
+__device__ __forceinline__ void getrf_steps(const SmallCtx &c, int p, v4d (&R0)[8], v4d (&R1)[8],
+                                            double *W1, const double *W2, double *raw, double *Ub)
+{
+    switch (p) {
+    case 0: getrf_step<0, W0>(c, R0, R1, W1, W2, raw, Ub); break;
+    case 1: getrf_step<1, W0>(c, R0, R1, W1, W2, raw, Ub); break;
+    case 2: getrf_step<2, W0>(c, R0, R1, W1, W2, raw, Ub); break;
+    case 3: getrf_step<3, W0>(c, R0, R1, W1, W2, raw, Ub); break;
+    case 4: getrf_step<4, W0>(c, R0, R1, W1, W2, raw, Ub); break;
+    case 5: getrf_step<5, W0>(c, R0, R1, W1, W2, raw, Ub); break;
+    default: getrf_step<6, W0>(c, R0, R1, W1, W2, raw, Ub); break;
+    }
+}
+
+template <bool W0>
+__device__ __forceinline__ void getrf_waves(SmallCtx c, const UnitDesc &u, double *W1, double *W2,
+                                            double *D, double *raw, double *Ub)
+{
+    const int n = c.n, nb = c.nb, w = c.w, li = c.li, lk = c.lk;
+    v4d R0[8], R1[8];  // loads first, then the edges
+    auto mask = [&](v4d &v, int i, int j) {
+        if (i >= nb - 1 || j >= nb - 1)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int r = 16 * i + li, k = 16 * j + 4 * e + lk;
+                v[e] = (r < n && k < n) ? v[e] : (r == k ? 1.0 : 0.0);
+            }
+    };
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+        load_blk16(R0[j], c.a, c.lda, n, w, j, li, lk);
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+        load_blk16(R1[j], c.a, c.lda, n, w + 4, j, li, lk);
+    if (n & 15)
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            mask(R0[j], w, j);
+    if (W0) {
+        put_diag16(c, W1, R0[0]);
+        put_raw16<1>(c, R0, raw);
+    }
+    if (n & 15)
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            mask(R1[j], w + 4, j);
+    lds_barrier();  // C
+    for (int p = 0;; p++) {
+        c.refresh();
+        if (W0)
+            getrf_diag(c, u, p, W1, W2, D + (p & 1) * BF_BLK);
+        lds_barrier();  // A
+        if (p + 1 < nb)
+            getrf_steps<W0>(c, p, R0, R1, W1, W2, raw, Ub);
+        if (w == (p & 3))
+            store_diag16<false>(c, p, D + (p & 1) * BF_BLK);
+        if (p + 1 == nb)
+            break;
+    }
+}
+
+__device__ __attribute__((always_inline)) inline void getrf_small(const UnitDesc &u, double *smem)
+{
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const SmallCtx c = {u.m,       (u.m + 15) >> 4, w, lane & 15, lane >> 4, lane, gp(u.c),
+                        (unsigned)__builtin_amdgcn_readfirstlane(u.ldc)};
+    double *W1 = smem, *W2 = W1 + BF_BLK, *D = W2 + BF_BLK;
+    double *raw = D + 2 * BF_BLK, *Ub = raw + 7 * BF_BLK;
+    __builtin_amdgcn_s_setprio(3);
+    if (w == 0)
+        getrf_waves<true>(c, u, W1, W2, D, raw, Ub);
+    else
+        getrf_waves<false>(c, u, W1, W2, D, raw, Ub);
     __builtin_amdgcn_s_setprio(0);
 }
 
@@ -2079,15 +2481,14 @@ constexpr int LDS_TRSM_SMALL = SMALL_MAX * 16 + 16 * 17;
 
 // Small GETRF/POTRF or CVT item (the only kinds k_batch_small runs), on NW
 // waves; a CVT item uses the first four.
-template <int NW = 4>
 __device__ __attribute__((always_inline)) inline void run_small_item(const UnitDesc &u, int it,
                                                                      double *smem)
 {
     if (u.op == OP_GETRF)
-        factor_small_blk<false, NW>(u, smem);
+        getrf_small(u, smem);
     else if (u.op == OP_POTRF)
-        factor_small_blk<true, NW>(u, smem);
-    else if (threadIdx.x < WG_THREADS)
+        potrf_small(u, smem);
+    else
         cvt_block(u, it, smem);
 }
 
@@ -2123,8 +2524,8 @@ __device__ __attribute__((always_inline)) inline void run_item(const UnitDesc &u
         default: break;
         }
         break;
-    case OP_GETRF: factor_small_blk<false>(u, smem); break;
-    case OP_POTRF: factor_small_blk<true>(u, smem); break;
+    case OP_GETRF: getrf_small(u, smem); break;
+    case OP_POTRF: potrf_small(u, smem); break;
     case OP_CVT: cvt_block(u, it, smem); break;
     case OP_TRINV: run_trinv_item(u, it, smem); break;
     default: break;

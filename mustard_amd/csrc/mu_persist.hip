@@ -104,8 +104,8 @@ constexpr int LDS_PERSIST_A = PERSIST_TRSM_MAX * 16 > TRINV_BLOCKS * 16 * 17
                                   ? PERSIST_TRSM_MAX * 16
                                   : TRINV_BLOCKS * 16 * 17;
 constexpr int LDS_PERSIST_B = LDS_GEMM > LDS_TRSM_SMALL ? LDS_GEMM : LDS_TRSM_SMALL;
-constexpr int LDS_PERSIST = LDS_PERSIST_A > LDS_PERSIST_B ? LDS_PERSIST_A : LDS_PERSIST_B;
-static_assert(LDS_PERSIST >= LDS_SMALL, "persistent LDS holds the small factorizations");
+constexpr int LDS_PERSIST_C = LDS_PERSIST_A > LDS_PERSIST_B ? LDS_PERSIST_A : LDS_PERSIST_B;
+constexpr int LDS_PERSIST = LDS_PERSIST_C > LDS_SMALL ? LDS_PERSIST_C : LDS_SMALL;
 
 // The kernel's LDS, at file scope so the item bodies below address it as LDS
 // without a pointer argument.
