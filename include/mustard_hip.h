@@ -128,13 +128,11 @@ int mu_dtrsm(void *stream, char side, char uplo, char transa, char diag, int m, 
 /* No counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  mu_dtrsm with the same arguments, meaning and result
- * (bit for bit), run at once on `stream`; the inverted diagonal blocks of a
- * triangle of order > 128 go to a fixed device array of
- * MU_NOALLOC_SCRATCH_BYTES per GPU (held until the process ends) instead of a
- * per-call allocation, so triangles of order <= 8192 are accepted and larger
- * ones rejected with MU_EINVAL.  Calls that overlap on one GPU share that
- * array and race; a stream being recorded into a DAG is refused
- * (MU_ESTATE).  Allocates no device memory. */
+ * (bit for bit), run at once on `stream`.  Triangles of order <= 8192 are
+ * accepted and larger ones rejected with MU_EINVAL; a stream being recorded
+ * into a DAG is refused (MU_ESTATE).  Allocates no device memory and keeps
+ * none (MU_NOALLOC_SCRATCH_BYTES, the size of a device array that earlier
+ * versions held, is defined for callers that read it). */
 #define MU_NOALLOC_SCRATCH_BYTES (1u << 21)
 #define MU_NOALLOC_MAX_ORDER 8192
 int mu_dtrsm_noalloc(void *stream, char side, char uplo, char transa, char diag, int m, int n,
@@ -222,9 +220,9 @@ int mu_exec_level_ops(mu_exec_t exec, int level, long long *counts);
  * MU_KERNEL_GEMM: k_batch_gemm, GEMM/SYRK blocks only; MU_KERNEL_SMALL:
  * k_batch_small, diagonal GETRF/POTRF of order <= 128 only; MU_KERNEL_TRSM: k_batch_trsm, 8-wave panel solves with
  * inverted diagonal blocks only; MU_KERNEL_TRSM_SMALL: k_batch_trsm_small,
- * panel solves of order <= 128 without inverted blocks only; MU_KERNEL_TRSM_256 /
- * MU_KERNEL_TRSM_512: k_batch_trsm_mid<256 / 512>, 4-wave panel solves with
- * inverted diagonal blocks of order <= 256 / 512 and the block inversions
+ * panel solves of order <= 128 only; MU_KERNEL_TRSM_256: k_batch_trsm_256, panel
+ * solves of order <= 256; MU_KERNEL_TRSM_512: k_batch_trsm_512, 4-wave panel
+ * solves with inverted diagonal blocks of order <= 512 and the block inversions
  * before them; MU_KERNEL_GEMM_NARROW: k_batch_gemm_narrow, GEMMs with at most
  * 16 output columns; MU_KERNEL_GEMM_LOW: k_batch_gemm_low, FP32 / BF16 updates
  * reading the converted panels, both operands k-contiguous; MU_KERNEL_CVT:

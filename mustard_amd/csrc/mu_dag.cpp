@@ -433,8 +433,9 @@ struct Builder {
             if (op.m <= o.trsm_max) {
                 UnitDesc d = base(op);
                 d.gm = 1;
-                d.gn = cdiv(op.n, TRSM_W);
-                if (op.m >= o.trsm_inv_min) {
+                d.gn = cdiv(op.n, 4 * TRSM_W);
+                if (op.m > TRSM_REG_MAX) {
+                    d.gn = cdiv(op.n, TRSM_W);
                     // the triangle's 16 x 16 diagonal blocks are inverted once,
                     // by a TRINV unit, for all panels of the solve
                     const int nblk = cdiv(op.m, 16), slot = (int)ws_doubles.size();
@@ -693,7 +694,7 @@ double item_cost_us(const UnitDesc &u)
     case OP_SYRK:
         return 3.0 + 2.0 * std::min(u.m, GEMM_BM) * std::min(u.n, GEMM_BN) * (double)u.k /
                          (0.8 * per_cu_flops);
-    case OP_TRSM: return 3.0 + (double)u.m * u.m * TRSM_W / (0.2 * per_cu_flops) + u.m * 0.05;
+    case OP_TRSM: return 3.0 + (double)u.m * u.m * TRSM_W / (0.25 * per_cu_flops);
     case OP_GETRF: return 3.0 + 2.0 * u.m * u.m * (double)u.m / 3.0 / (0.05 * per_cu_flops);
     case OP_POTRF: return 3.0 + u.m * u.m * (double)u.m / 3.0 / (0.05 * per_cu_flops);
     case OP_TRINV: return 5.0;

@@ -79,34 +79,40 @@ __global__ __launch_bounds__(WG_THREADS) void k_batch_gemm_narrow(const UnitDesc
     run_gemm_narrow_item(d, (int)(item - d.item_base), smem);
 }
 
-// Panel solves of order <= SMALL_MAX (inside nested diagonal factorizations).
-__global__ __launch_bounds__(WG_THREADS) void k_batch_trsm_small(const UnitDesc *units,
-                                                                 const uint32_t *item_unit,
-                                                                 const uint32_t *items)
+// Panel solves of order <= SMALL_MAX (inside nested diagonal factorizations)
+// and of order <= TRSM_REG_MAX, at most 200 registers per lane as
+// k_batch_small, so they start beside three GEMM workgroups.
+__global__ __launch_bounds__(WG_THREADS) __attribute__((amdgpu_num_vgpr(100))) void
+k_batch_trsm_small(const UnitDesc *units, const uint32_t *item_unit, const uint32_t *items)
 {
-    __shared__ double smem[LDS_TRSM_SMALL];
+    __shared__ __align__(16) double smem[LDS_TRSM_REG_SMALL];
     const uint32_t item = items[blockIdx.x];
     const UnitDesc d = units[item_unit[item]];
-    run_trsm_small_item(d, (int)(item - d.item_base), smem);
+    run_trsm_reg_item<8>(d, (int)(item - d.item_base), smem);
 }
 
-// Panel solves with inverted diagonal blocks of order <= NMAX, and the TRINV
-// items before them, on 4 waves and at most NMAX * 128 bytes of LDS
-// (k_batch_trsm_256: 34 KB, k_batch_trsm_512: 64 KB), so GEMM workgroups keep
-// running beside them on the same CU.
-template <int NMAX>
-__global__ __launch_bounds__(WG_THREADS) void k_batch_trsm_mid(const UnitDesc *units,
+__global__ __launch_bounds__(WG_THREADS) __attribute__((amdgpu_num_vgpr(100))) void
+k_batch_trsm_256(const UnitDesc *units, const uint32_t *item_unit, const uint32_t *items)
+{
+    __shared__ __align__(16) double smem[LDS_TRSM_REG];
+    const uint32_t item = items[blockIdx.x];
+    const UnitDesc d = units[item_unit[item]];
+    run_trsm_reg_item<16>(d, (int)(item - d.item_base), smem);
+}
+
+// Panel solves with inverted diagonal blocks of order <= 512, and the TRINV
+// items before them, on 4 waves and 64 KB of LDS (trsm_max above 256 only).
+__global__ __launch_bounds__(WG_THREADS) void k_batch_trsm_512(const UnitDesc *units,
                                                                const uint32_t *item_unit,
                                                                const uint32_t *items)
 {
-    constexpr int LDSD = NMAX * 16 > TRINV_BLOCKS * 16 * 17 ? NMAX * 16 : TRINV_BLOCKS * 16 * 17;
-    __shared__ double smem[LDSD];
+    __shared__ double smem[512 * 16];
     const uint32_t item = items[blockIdx.x];
     const UnitDesc d = units[item_unit[item]];
     if (d.op == OP_TRINV)
         run_trinv_item(d, (int)(item - d.item_base), smem);
     else
-        run_trsm_inv_item<4, NMAX>(d, (int)(item - d.item_base), smem);
+        run_trsm_inv_item<4, 512>(d, (int)(item - d.item_base), smem);
 }
 
 const void *level_kernel(int kind)
@@ -118,8 +124,8 @@ const void *level_kernel(int kind)
     case LEVEL_GEMM_NARROW: return reinterpret_cast<const void *>(k_batch_gemm_narrow);
     case LEVEL_GEMM_LOW: return reinterpret_cast<const void *>(k_batch_gemm_low);
     case LEVEL_CVT: return reinterpret_cast<const void *>(k_batch_cvt);
-    case LEVEL_TRSM_256: return reinterpret_cast<const void *>(k_batch_trsm_mid<256>);
-    case LEVEL_TRSM_512: return reinterpret_cast<const void *>(k_batch_trsm_mid<512>);
+    case LEVEL_TRSM_256: return reinterpret_cast<const void *>(k_batch_trsm_256);
+    case LEVEL_TRSM_512: return reinterpret_cast<const void *>(k_batch_trsm_512);
     default: return generic_kernel(kind);
     }
 }

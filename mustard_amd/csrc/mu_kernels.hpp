@@ -25,10 +25,9 @@ enum LevelKernel : char {
 
 constexpr int TRSM_KERNEL_WAVES = 8;  // k_batch_trsm: two waves per SIMD
 
-// Largest panel-solve triangle with inverted diagonal blocks the persistent
-// kernel runs (its LDS holds the panel and the TRINV staging, 34 KB); larger
-// solves are nested by the lowering.
-constexpr int PERSIST_TRSM_MAX = 256;
+// Largest panel-solve triangle the persistent kernel runs; larger solves are
+// nested by the lowering.
+constexpr int PERSIST_TRSM_MAX = TRSM_REG_MAX;
 
 // Kernel handle and block size of a graph node of kind `kind` (mu_kern.hip).
 const void *level_kernel(int kind);

@@ -843,166 +843,7 @@ __device__ __attribute__((always_inline)) inline void gemm_block_lowk128(const U
 constexpr int LDS_GEMM_LOWK128 = 2 * 256 * (64 + 8) * 2 / 8;
 
 // ---------------------------------------------------------------------------
-// Panel triangular solve.  Solves T Y = Z in place for one panel of up to 16
-// right-hand sides, T lower triangular of order n <= TRSM_NMAX:
-//   left-lower-unit   X = L^-1 B  : T = L,   Z = B (columns)
-//   right-upper       X = B U^-1  : T = U^T, Z = B^T (rows of B)
-//   right-lower-trans X = B L^-T  : T = L,   Z = B^T (rows of B)
-// With REV the row order of T and Z is reversed, which turns an upper
-// triangular solve (back substitution) into the same lower-triangular form.
-// Z is scaled by alpha on load.  The panel lives in LDS; each 16-row step solves its diagonal block with one
-// thread per right-hand side and updates the rows below with FP64 MFMA.
-// ---------------------------------------------------------------------------
-template <bool TT, bool ZR, bool UNIT, bool REV, int NMAX = TRSM_NMAX>
-__device__ __attribute__((always_inline)) inline void trsm_panel(const UnitDesc &u, int panel, double *smem)
-{
-    // NMAX: largest triangle the caller's LDS holds (TRSM_NMAX in the generic
-    // kernel, SMALL_MAX in k_batch_trsm_small)
-    const int n = u.m, p0 = panel * TRSM_W, w = min(TRSM_W, u.n - p0);
-    const int np = (n + 15) & ~15;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    double *Y = smem;              // [np][16]
-    double *Td = smem + NMAX * 16; // [16][17]
-    const MU_G double *t = gp(u.a);
-    const size_t ldt = u.lda, ldz = u.ldc;
-    MU_G double *z = gp(u.c);
-    const double alpha = u.alpha;
-    // 32-bit offsets with 24-bit multiplies (full rate, unlike 64-bit
-    // products): the lowering guarantees (n + 1) * ldt < 2^31 for triangles
-    const unsigned ldt32 = (unsigned)ldt;
-    auto tv = [&](int r, int c) -> double {
-        if (REV) {
-            r = n - 1 - r;
-            c = n - 1 - c;
-        }
-        const unsigned off = TT ? (unsigned)c + __umul24((unsigned)r, ldt32)
-                                : (unsigned)r + __umul24((unsigned)c, ldt32);
-        return t[off];
-    };
-    auto zp = [&](int r, int c) -> MU_G double * {
-        if (REV)
-            r = n - 1 - r;
-        return ZR ? z + (p0 + c) + r * ldz : z + r + (p0 + c) * ldz;
-    };
-
-    for (int idx = tid; idx < np * 16; idx += WG_THREADS) {
-        int r, c;
-        if (ZR) {
-            c = idx & 15;
-            r = idx >> 4;
-        } else {
-            r = idx % np;
-            c = idx / np;
-        }
-        Y[r * 16 + c] = (r < n && c < w) ? alpha * *zp(r, c) : 0.0;
-    }
-    lds_barrier();
-
-    // Each 16-row step jb: stage the diagonal block (reciprocals of its
-    // diagonal in place of the entries, so the solve multiplies), solve it
-    // with one thread per right-hand side, then update the rows below,
-    // Y[rb] -= T[rb, jb] Y[jb], with FP64 MFMA.  The triangle fragments of
-    // step jb+16 are loaded during step jb, row block by row block right
-    // after that block's MFMAs, so they are consumed in the order they were
-    // issued and at most 64 loads per lane are in flight (the hardware's
-    // in-order vector-memory counter tracks 63).
-    const int li = lane & 15, lk = lane >> 4;
-    const int r16 = tid >> 4, c16 = tid & 15;
-    constexpr int MAXB = NMAX / 64 > 0 ? NMAX / 64 : 1;
-    // Loads are unconditional, from addresses clamped into the triangle;
-    // values outside it are zeroed where they are used (see the header of
-    // the GEMM loaders for why no load sits behind a branch).
-    auto load_diag = [&](int jb) -> double {
-        return tv(min(jb + r16, n - 1), min(jb + c16, n - 1));
-    };
-    auto load_block = [&](double (&f)[4], int jb, int i) {
-        const int rb = jb + 16 + 16 * wave + 64 * i;
-#pragma unroll
-        for (int kk = 0; kk < 4; kk++)
-            f[kk] = tv(min(rb + li, n - 1), min(jb + 4 * kk + lk, n - 1));
-    };
-    auto step = [&](int jb, double dv, const double (&fa)[MAXB][4], double &dn,
-                    double (&fn)[MAXB][4]) {
-        dv = (jb + r16 < n && c16 <= r16) ? dv : 0.0;
-        if (!UNIT && c16 == r16 && jb + r16 < n)
-            dv = 1.0 / dv;
-        Td[r16 * 17 + c16] = dv;
-        lds_barrier();
-        if (tid < 16) {
-            const int nb = min(16, n - jb);
-            double y[16];
-#pragma unroll
-            for (int r = 0; r < 16; r++)
-                y[r] = Y[(jb + r) * 16 + tid];
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                if (r < nb) {
-                    double s = y[r];
-#pragma unroll
-                    for (int q = 0; q < r; q++)
-                        s -= Td[r * 17 + q] * y[q];
-                    if (!UNIT)
-                        s *= Td[r * 17 + r];
-                    y[r] = s;
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 16; r++)
-                if (r < nb)
-                    Y[(jb + r) * 16 + tid] = y[r];
-        }
-        lds_barrier();
-        dn = load_diag(jb + 16);
-        double fb[4];
-#pragma unroll
-        for (int kk = 0; kk < 4; kk++)
-            fb[kk] = Y[(jb + 4 * kk + lk) * 16 + li];
-#pragma unroll
-        for (int i = 0; i < MAXB; i++) {
-            const int rb = jb + 16 + 16 * wave + 64 * i;
-            if (rb < np) {
-                v4d acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-                for (int kk = 0; kk < 4; kk++) {
-                    const bool in = rb + li < n && jb + 4 * kk + lk < n;
-                    acc = mfma_f64(in ? fa[i][kk] : 0.0, fb[kk], acc);
-                }
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    Y[(rb + 4 * e + lk) * 16 + li] -= acc[e];
-            }
-            load_block(fn[i], jb + 16, i);
-        }
-        lds_barrier();
-    };
-    double fa0[MAXB][4], fa1[MAXB][4];
-    double d0 = load_diag(0), d1 = 0.0;
-#pragma unroll
-    for (int i = 0; i < MAXB; i++)
-        load_block(fa0[i], 0, i);
-    for (int jb = 0; jb < n; jb += 32) {
-        step(jb, d0, fa0, d1, fa1);
-        if (jb + 16 >= n)
-            break;
-        step(jb + 16, d1, fa1, d0, fa0);
-    }
-
-    for (int idx = tid; idx < np * 16; idx += WG_THREADS) {
-        int r, c;
-        if (ZR) {
-            c = idx & 15;
-            r = idx >> 4;
-        } else {
-            r = idx % np;
-            c = idx / np;
-        }
-        if (r < n && c < w)
-            *zp(r, c) = Y[r * 16 + c];
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Inverted diagonal blocks.  For a triangle T of order n > SMALL_MAX (read in
+// Inverted diagonal blocks.  For a triangle T of order n > TRSM_REG_MAX (read in
 // the canonical lower form the panel solve uses: flags TT, UNIT, REV as in
 // trsm_panel), item `it` inverts diagonal blocks 16*it .. 16*it+15 of 16 x 16
 // and stores inv(T_jj) row-major at c + 256 j.  Rows and columns of the last
@@ -1059,9 +900,10 @@ __device__ __attribute__((always_inline)) inline void trinv_blocks(const UnitDes
 }
 
 // ---------------------------------------------------------------------------
-// Panel triangular solve with inverted diagonal blocks (triangles of order
-// n > SMALL_MAX; the TRINV unit before it left inv(T_jj) at u.b).  Same
-// problem and flags as trsm_panel.  Step jb: every wave forms the solved
+// Panel triangular solve in LDS with inverted diagonal blocks (triangles of
+// order n > TRSM_REG_MAX, made only where mu_exec_opts_t.trsm_max asks for
+// them; the TRINV unit before it left inv(T_jj) at u.b).  Same problem and
+// flags as trsm_panel_reg, panels of 16 right-hand sides.  Step jb: every wave forms the solved
 // block X_jb = inv(T_jj) Y_jb with four MFMAs -- the result's register layout
 // is exactly the B operand of the update MFMAs, so it never goes back
 // through LDS -- wave 0 stores it to Z, and each wave updates its row blocks
@@ -1895,11 +1737,316 @@ __device__ __attribute__((always_inline)) inline void getrf_small(const UnitDesc
     __builtin_amdgcn_s_setprio(0);
 }
 
+// ---------------------------------------------------------------------------
+// Panel triangular solve, T Y = alpha Z in place, T lower triangular of order
+// n <= TRSM_REG_MAX:
+//   left-lower-unit   X = L^-1 B  : T = L,   Z = B (columns)
+//   right-upper       X = B U^-1  : T = U^T, Z = B^T (rows of B)
+//   right-lower-trans X = B L^-T  : T = L,   Z = B^T (rows of B)
+// With F_REV the row order of T and Z is reversed, which turns an upper
+// triangular solve (back substitution) into the same lower-triangular form.
+//
+// What bounds it: beside the other panel work it is on the chain to the next
+// diagonal tile, and over a whole panel it is the matrix pipe.  Each wave
+// owns 16 right-hand sides and keeps them in registers in the MFMA result
+// layout (element e of block i: row 16 i + 4 e + lk, column li), which is the
+// MFMA B operand, so a solve is a stream of MFMAs: X_j = inv(T_jj) Y_j, then
+// Y_i -= T_ij X_j for the blocks below.  A work item is 64 right-hand sides
+// (four waves).  The blocks T_ij below the diagonal stream through a ring in
+// LDS in the order of use, copied by the waves in turn (global_load_lds,
+// groups of four blocks, TRSM_RING - 1 groups ahead, one barrier per group):
+// read by each wave for itself four blocks ahead, the stream was bound by
+// memory latency (order 250: 48 us).  The workgroup first inverts all 16 x 16
+// diagonal blocks at once, one block per group of 16 lanes, so no inversion
+// kernel runs before it.  One node of the Cholesky at n = 7007, against a
+// panel of 16 right-hand sides per workgroup in LDS (a barrier per 16 rows,
+// four waves sharing each panel): order 125 28 -> 14 us, order 250 35 us
+// after an inversion kernel of 10 us -> 38 us; N = 24000 LU 166 -> 152 ms.
+//
+// Strides are run-time values, so one body serves every side, triangle and
+// transposition; blocks past the triangle compute on whatever the ring holds
+// and are never stored.
+// ---------------------------------------------------------------------------
+// Groups of four T blocks in the ring: as many as keep the workgroup beside
+// three GEMM workgroups of 32 KB with 16 inverses (34 KB), beside four with 8
+// (four groups there: N = 24000 Cholesky 80.4 -> 78.8 ms with two).
+template <int NB>
+constexpr int TRSM_RING = NB > 8 ? 3 : 2;
+
+template <class T>
+__device__ __forceinline__ T *uniform_ptr(T *p)
+{
+    const unsigned long long v = (unsigned long long)p;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
+    return (T *)(((unsigned long long)hi << 32) | lo);
+}
+
+// column li of the inverse of a lower 16 x 16 block, lane li holding row li in
+// x and 1 / its diagonal in rd: row C to W[C * BF_LD]
+template <int C>
+__device__ __forceinline__ void tri_inv16(double (&z)[16], const double (&x)[16], double rd,
+                                          double *W)
+{
+    if constexpr (C < 16) {
+        z[C] *= bcast16<C>(rd);
+        W[C * BF_LD] = z[C];
+        fms_lane<C + 1>(z, x[C], z[C]);
+        tri_inv16<C + 1>(z, x, rd, W);
+    }
+}
+
+// The T blocks below the diagonal in the order of use, column by column:
+// block S of column J, row I.
+template <int NB>
+struct TrsmOrder {
+    static constexpr int first(int j) { return j * (2 * NB - j - 1) / 2; }
+    static constexpr int count = NB * (NB - 1) / 2, groups = (count + 3) / 4;
+};
+
+// Copies of this wave's block of each group of four into the ring.
+template <int NB>
+struct TrsmFeed {
+    const MU_G double *t;
+    unsigned ldt;
+    int n, nb, lane;
+    bool tt, rev;
+    double *ring;  // this wave's slot of group 0
+    int i, j;      // the block copied next
+    __device__ __forceinline__ void copy(int g)
+    {
+        // T's block (i, j) in memory: rows from r0, columns from c0 (rev:
+        // counted from the end, so it lies there mirrored).  Blocks past the
+        // triangle take a block inside it.
+        const int ic = min(i, nb - 1), jc = min(j, nb - 2);
+        const int r0 = rev ? n - 16 - 16 * ic : 16 * ic, c0 = rev ? n - 16 - 16 * jc : 16 * jc;
+        double *d = ring + (g % TRSM_RING<NB>) * 4 * 256;
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            const int a = 8 * q + (lane >> 3), b = lane & 7;
+            // not transposed: column a, rows 2 b, 2 b + 1 at [a * 16 + 2 b];
+            // rows past n are still inside the triangle's storage (column c0
+            // + a is not the last one).  Transposed: row a, columns in
+            // 16-byte chunks, chunk c at c ^ ((a / 2) % 8); rows clamped.
+            const long long off =
+                tt ? (long long)max(min(r0 + a, n - 1), 0) * ldt + c0 + 2 * (b ^ ((a >> 1) & 7))
+                   : (long long)(c0 + a) * ldt + r0 + 2 * b;
+            __builtin_amdgcn_global_load_lds((const MU_G unsigned *)(t + off),
+                                             (MU_LDS unsigned *)(d + 128 * q), 16, 0, 0);
+        }
+        i += 4;
+        wrap();
+    }
+    // to the column the block belongs to (past the last column: any)
+    __device__ __forceinline__ void wrap()
+    {
+        while (i >= NB && j < NB - 1) {
+            j++;
+            i += j + 1 - NB;
+        }
+    }
+};
+
+// Start of group G: its copies have landed in every wave's slot; then the
+// copies TRSM_RING - 1 groups on (into the slots of group G - 1, which every
+// wave has read).
+template <int NB, int G>
+__device__ __forceinline__ void trsm_group(TrsmFeed<NB> &feed)
+{
+    constexpr int last = TrsmOrder<NB>::groups - 1;
+    constexpr int R = TRSM_RING<NB>, ahead = (G + R - 2 < last ? G + R - 2 : last) - G;
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * ahead) : "memory");
+    if constexpr (G + R - 1 <= last)
+        feed.copy(G + R - 1);
+}
+
+// Y[I ..] -= T[I .., J] X_J (nx = -X_J).
+template <int NB, int J, int I>
+__device__ __forceinline__ void trsm_below(v4d (&Y)[NB], const double *ring, const int (&lo)[4],
+                                           const v4d &nx, TrsmFeed<NB> &feed)
+{
+    if constexpr (I < NB) {
+        constexpr int S = TrsmOrder<NB>::first(J) + I - J - 1;
+        if constexpr (S % 4 == 0)
+            trsm_group<NB, S / 4>(feed);
+        const double *b = ring + (S / 4 % TRSM_RING<NB> * 4 + S % 4) * 256;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            Y[I] = mfma_f64(b[lo[e]], nx[e], Y[I]);
+        trsm_below<NB, J, I + 1>(Y, ring, lo, nx, feed);
+    }
+}
+// Columns J ..: X_J replaces Y_J.  The last block's rows past the triangle
+// (rlast: the rows below this lane's first that are inside) were updated with
+// rows of T that are not its own; they are zero as its inverse meets them.
+template <int NB, int J>
+__device__ __forceinline__ void trsm_columns(v4d (&Y)[NB], const double *W, const double *ring,
+                                             const int (&lo)[4], int nb, int rlast,
+                                             TrsmFeed<NB> &feed)
+{
+    if constexpr (J < NB) {
+        if (J >= nb)
+            return;
+        if (J == nb - 1)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                Y[J][e] = 4 * e < rlast ? Y[J][e] : 0.0;
+        v4d x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            x = mfma_f64(W[J * BF_BLK + 4 * e], Y[J][e], x);
+        Y[J] = x;
+        if (J + 1 < nb) {
+            const v4d nx = -x;
+            trsm_below<NB, J, J + 1>(Y, ring, lo, nx, feed);
+        }
+        trsm_columns<NB, J + 1>(Y, W, ring, lo, nb, rlast, feed);
+    }
+}
+
+template <int NB>
+__device__ __attribute__((always_inline)) inline void trsm_panel_reg(const UnitDesc &u, int it,
+                                                                     double *smem)
+{
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = __builtin_amdgcn_readfirstlane(u.m), nb = (n + 15) >> 4;
+    const int ncol = __builtin_amdgcn_readfirstlane(u.n);
+    const int flags = __builtin_amdgcn_readfirstlane(u.flags);
+    const bool rev = flags & F_REV, tt = flags & F_T_TRANS, zr = flags & F_Z_ROWS;
+    const unsigned ldt = __builtin_amdgcn_readfirstlane(u.lda);
+    const unsigned ldz = __builtin_amdgcn_readfirstlane(u.ldc);
+    const MU_G double *t = gp(uniform_ptr(u.a));
+    MU_G double *z = gp(uniform_ptr(u.c));
+    const double alpha = u.alpha;
+    double *ring = smem + NB * BF_BLK;
+    // T(r, c) at t[r rs + c cs], Z(r, c) at z[r zrs + c zcs], rows (and T's
+    // columns) counted from the end with rev
+    const unsigned rs = tt ? ldt : 1, cs = tt ? 1 : ldt;
+    const unsigned zrs = zr ? ldz : 1, zcs = zr ? 1 : ldz;
+
+    TrsmFeed<NB> feed = {t, ldt, n, nb, lane, tt, rev, ring + wave * 256, 1 + wave, 0};
+    feed.wrap();
+    if (nb > 1)
+#pragma unroll
+        for (int g = 0; g < TRSM_RING<NB> - 1; g++)
+            if (g < TrsmOrder<NB>::groups)
+                feed.copy(g);
+
+    // ---- inverses of the diagonal blocks, block wave + 4 lk on this group
+    {
+        const int jb = min(wave + 4 * lk, nb - 1);
+        const int r = 16 * jb + li, rc = min(r, n - 1);
+        double x[16], v[16];
+        auto at = [&](int rr, int cc) -> double {
+            const size_t a = rev ? n - 1 - rr : rr, b = rev ? n - 1 - cc : cc;
+            return t[a * rs + b * cs];
+        };
+#pragma unroll
+        for (int c = 0; c < 16; c++)
+            x[c] = at(rc, min(16 * jb + c, n - 1));
+        const double dv = at(rc, rc);
+#pragma unroll
+        for (int c = 0; c < 16; c++) {
+            x[c] = r < n ? x[c] : 0.0;
+            v[c] = c == li ? 1.0 : 0.0;
+        }
+        const double rd = ((flags & F_UNIT) || r >= n) ? 1.0 : 1.0 / dv;
+        tri_inv16<0>(v, x, rd, smem + jb * BF_BLK + li);
+    }
+
+    // ---- the panel (rows past n: the last row).  A wave without right-hand
+    // sides repeats the last panel's and stores nothing.
+    const int p0 = (it * 4 + wave) * TRSM_W, w = min(TRSM_W, ncol - p0);
+    const int pc = min(p0, (ncol - 1) / TRSM_W * TRSM_W), lic = min(li, ncol - 1 - pc);
+    const int nlast = n - 16 * (nb - 1);
+    MU_G double *zb = z + (size_t)pc * zcs;
+    // row 16 i + 4 e + lk, column lic: a uniform part and this lane's
+    const unsigned zl = (rev ? 3 - lk : lk) * zrs + lic * zcs;
+    auto zrow = [&](int r) -> size_t {  // of rows r .. r + 3, the lowest address
+        return (size_t)(rev ? n - 4 - r : r) * zrs;
+    };
+    v4d Y[NB];
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+        Y[i] = v4d{0.0, 0.0, 0.0, 0.0};
+        if (i < nb - 1) {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                Y[i][e] = (zb + zrow(16 * i + 4 * e))[zl];
+        } else if (i == nb - 1) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int r = min(4 * e + lk, nlast - 1) + 16 * i;
+                Y[i][e] = zb[(size_t)(rev ? n - 1 - r : r) * zrs + lic * (size_t)zcs];
+            }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NB; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            Y[i][e] *= alpha;
+    lds_barrier();  // the inverses
+
+    // element (li, 4 e + lk) of a ring block
+    int lo[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int r = rev ? 15 - li : li, c = rev ? 15 - 4 * e - lk : 4 * e + lk;
+        lo[e] = tt ? r * 16 + (((c >> 1) ^ ((r >> 1) & 7)) << 1) + (c & 1) : c * 16 + r;
+    }
+    trsm_columns<NB, 0>(Y, smem + li * BF_LD + lk, ring, lo, nb, nlast - lk, feed);
+
+    if (li < w)
+#pragma unroll
+        for (int i = 0; i < NB; i++) {
+            if (i < nb - 1) {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    (zb + zrow(16 * i + 4 * e))[zl] = Y[i][e];
+            } else if (i == nb - 1) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int r = 16 * i + 4 * e + lk;
+                    if (r < n)
+                        zb[(size_t)(rev ? n - 1 - r : r) * zrs + li * (size_t)zcs] = Y[i][e];
+                }
+            }
+        }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // copies past the triangle have landed
+}
+constexpr int LDS_TRSM_REG = 16 * BF_BLK + TRSM_RING<16> * 1024;       // inverses of order TRSM_REG_MAX
+constexpr int LDS_TRSM_REG_SMALL = 8 * BF_BLK + TRSM_RING<8> * 1024;  // ... of order SMALL_MAX
+
+// TRSM item of a triangle of order <= TRSM_REG_MAX; MAXNB: the most 16-blocks
+// the caller's LDS holds inverses for (8 or 16).  The block count is rounded
+// up to an instance (a block past the triangle costs its MFMAs).
+template <int MAXNB>
+__device__ __attribute__((always_inline)) inline void run_trsm_reg_item(const UnitDesc &u, int it,
+                                                                        double *smem)
+{
+    const int nb = (__builtin_amdgcn_readfirstlane(u.m) + 15) >> 4;
+    if (nb <= 2)
+        trsm_panel_reg<2>(u, it, smem);
+    else if (nb <= 4)
+        trsm_panel_reg<4>(u, it, smem);
+    else if (nb <= 6)
+        trsm_panel_reg<6>(u, it, smem);
+    else if (MAXNB == 8 || nb <= 8)
+        trsm_panel_reg<8>(u, it, smem);
+    else if (nb <= 12)
+        trsm_panel_reg<MAXNB == 8 ? 8 : 12>(u, it, smem);
+    else
+        trsm_panel_reg<MAXNB == 8 ? 8 : 16>(u, it, smem);
+}
+
 // LDS (doubles) one workgroup needs for any item.
 constexpr int LDS_GEMM = LDS_GEMM_DMA;
 static_assert(2 * (LDS_I > LDS_K ? LDS_I : LDS_K) * 2 <= LDS_GEMM, "gemm_block: 2 operands x 2 buffers");
 constexpr int LDS_NARROW = 4 * 4 * 4 * 64 / 2 + 1;  // the narrow GEMMs' partial tiles and a flag
-constexpr int LDS_TRSM = TRSM_NMAX * 16 + 16 * 17;
+constexpr int LDS_TRSM = TRSM_NMAX * 16;
 constexpr int LDS_SMALL = LDS_SMALL_BLK;
 static_assert(TRINV_BLOCKS * 16 * 17 <= LDS_TRSM, "TRINV staging fits the generic LDS");
 static_assert(TRINV_BLOCKS * 16 == WG_THREADS, "TRINV: one thread per block column");
@@ -2420,7 +2567,7 @@ __device__ __attribute__((always_inline)) inline void cvt_block(const UnitDesc &
 }
 
 // TRSM item with inverted diagonal blocks on NW waves (k_batch_trsm,
-// k_batch_trsm_mid).
+// k_batch_trsm_512).
 template <int NW, int NMAX = TRSM_NMAX>
 __device__ __attribute__((always_inline)) inline void run_trsm_inv_item(const UnitDesc &u, int it,
                                                                         double *smem)
@@ -2456,29 +2603,6 @@ __device__ __attribute__((always_inline)) inline void run_trinv_item(const UnitD
     }
 }
 
-// Panel solve of a triangle of order <= SMALL_MAX without inverted blocks
-// (k_batch_trsm_small: the panel in 18.5 KB of LDS).
-__device__ __attribute__((always_inline)) inline void run_trsm_small_item(const UnitDesc &u, int it,
-                                                                          double *smem)
-{
-    switch ((u.flags >> 3) & 0x27) {  // T_TRANS, Z_ROWS, UNIT, REV
-#define MU_TRSM_SMALL_CASE(bits)                                                           \
-    case bits:                                                                             \
-        trsm_panel<(bits & 1) != 0, (bits & 2) != 0, (bits & 4) != 0, (bits & 0x20) != 0, \
-                   SMALL_MAX>(u, it, smem);                                                \
-        break;
-        MU_TRSM_SMALL_CASE(0x00) MU_TRSM_SMALL_CASE(0x01) MU_TRSM_SMALL_CASE(0x02)
-        MU_TRSM_SMALL_CASE(0x03) MU_TRSM_SMALL_CASE(0x04) MU_TRSM_SMALL_CASE(0x05)
-        MU_TRSM_SMALL_CASE(0x06) MU_TRSM_SMALL_CASE(0x07) MU_TRSM_SMALL_CASE(0x20)
-        MU_TRSM_SMALL_CASE(0x21) MU_TRSM_SMALL_CASE(0x22) MU_TRSM_SMALL_CASE(0x23)
-        MU_TRSM_SMALL_CASE(0x24) MU_TRSM_SMALL_CASE(0x25) MU_TRSM_SMALL_CASE(0x26)
-        MU_TRSM_SMALL_CASE(0x27)
-#undef MU_TRSM_SMALL_CASE
-    default: break;
-    }
-}
-constexpr int LDS_TRSM_SMALL = SMALL_MAX * 16 + 16 * 17;
-
 // Small GETRF/POTRF or CVT item (the only kinds k_batch_small runs), on NW
 // waves; a CVT item uses the first four.
 __device__ __attribute__((always_inline)) inline void run_small_item(const UnitDesc &u, int it,
@@ -2506,23 +2630,10 @@ __device__ __attribute__((always_inline)) inline void run_item(const UnitDesc &u
         break;
     case OP_SYRK: run_gemm_item(u, it, smem); break;
     case OP_TRSM:
-        switch ((u.flags >> 3) & 0x67) {  // T_TRANS, Z_ROWS, UNIT, REV, INV
-#define MU_TRSM_CASE(bits)                                                                      \
-    case bits:                                                                                  \
-        trsm_panel<(bits & 1) != 0, (bits & 2) != 0, (bits & 4) != 0, (bits & 0x20) != 0>(     \
-            u, it, smem);                                                                       \
-        break;                                                                                  \
-    case bits | 0x40:                                                                           \
-        trsm_panel_inv<(bits & 1) != 0, (bits & 2) != 0, (bits & 4) != 0, (bits & 0x20) != 0>( \
-            u, it, smem);                                                                       \
-        break;
-            MU_TRSM_CASE(0x00) MU_TRSM_CASE(0x01) MU_TRSM_CASE(0x02) MU_TRSM_CASE(0x03)
-            MU_TRSM_CASE(0x04) MU_TRSM_CASE(0x05) MU_TRSM_CASE(0x06) MU_TRSM_CASE(0x07)
-            MU_TRSM_CASE(0x20) MU_TRSM_CASE(0x21) MU_TRSM_CASE(0x22) MU_TRSM_CASE(0x23)
-            MU_TRSM_CASE(0x24) MU_TRSM_CASE(0x25) MU_TRSM_CASE(0x26) MU_TRSM_CASE(0x27)
-#undef MU_TRSM_CASE
-        default: break;
-        }
+        if (u.flags & F_INV)
+            run_trsm_inv_item<4>(u, it, smem);
+        else
+            run_trsm_reg_item<16>(u, it, smem);
         break;
     case OP_GETRF: getrf_small(u, smem); break;
     case OP_POTRF: potrf_small(u, smem); break;

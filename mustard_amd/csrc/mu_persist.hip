@@ -97,15 +97,9 @@ struct DevAtom {
 
 // Item bodies the persistent kernel runs.  The lowering for this mode keeps
 // every item within them: GEMM/SYRK blocks, narrow GEMMs, GETRF/POTRF/CVT of
-// order <= SMALL_MAX, panel solves with inverted diagonal blocks of order <=
-// PERSIST_TRSM_MAX (and their TRINV items), plain panel solves of order <=
-// SMALL_MAX.
-constexpr int LDS_PERSIST_A = PERSIST_TRSM_MAX * 16 > TRINV_BLOCKS * 16 * 17
-                                  ? PERSIST_TRSM_MAX * 16
-                                  : TRINV_BLOCKS * 16 * 17;
-constexpr int LDS_PERSIST_B = LDS_GEMM > LDS_TRSM_SMALL ? LDS_GEMM : LDS_TRSM_SMALL;
-constexpr int LDS_PERSIST_C = LDS_PERSIST_A > LDS_PERSIST_B ? LDS_PERSIST_A : LDS_PERSIST_B;
-constexpr int LDS_PERSIST = LDS_PERSIST_C > LDS_SMALL ? LDS_PERSIST_C : LDS_SMALL;
+// order <= SMALL_MAX, panel solves of order <= PERSIST_TRSM_MAX.
+constexpr int LDS_PERSIST_A = LDS_GEMM > LDS_TRSM_REG ? LDS_GEMM : LDS_TRSM_REG;
+constexpr int LDS_PERSIST = LDS_PERSIST_A > LDS_SMALL ? LDS_PERSIST_A : LDS_SMALL;
 
 // The kernel's LDS, at file scope so the item bodies below address it as LDS
 // without a pointer argument.
@@ -125,20 +119,10 @@ __device__ __noinline__ void persist_gemm_narrow(const UnitDesc *ud, int it)
     const UnitDesc d = *ud;
     run_gemm_narrow_item(d, it, p_smem);
 }
-__device__ __noinline__ void persist_trsm_inv(const UnitDesc *ud, int it)
+__device__ __noinline__ void persist_trsm(const UnitDesc *ud, int it)
 {
     const UnitDesc d = *ud;
-    run_trsm_inv_item<4, PERSIST_TRSM_MAX>(d, it, p_smem);
-}
-__device__ __noinline__ void persist_trsm_small(const UnitDesc *ud, int it)
-{
-    const UnitDesc d = *ud;
-    run_trsm_small_item(d, it, p_smem);
-}
-__device__ __noinline__ void persist_trinv(const UnitDesc *ud, int it)
-{
-    const UnitDesc d = *ud;
-    run_trinv_item(d, it, p_smem);
+    run_trsm_reg_item<16>(d, it, p_smem);
 }
 __device__ __noinline__ void persist_small(const UnitDesc *ud, int it)
 {
@@ -156,13 +140,7 @@ __device__ __forceinline__ void run_persist_item(const UnitDesc *ud, int op, int
             persist_gemm(ud, it);
         break;
     case OP_SYRK: persist_gemm(ud, it); break;
-    case OP_TRSM:
-        if (flags & F_INV)
-            persist_trsm_inv(ud, it);
-        else
-            persist_trsm_small(ud, it);
-        break;
-    case OP_TRINV: persist_trinv(ud, it); break;
+    case OP_TRSM: persist_trsm(ud, it); break;
     default: persist_small(ud, it); break;
     }
 }

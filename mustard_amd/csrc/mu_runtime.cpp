@@ -475,10 +475,10 @@ static int exec_build(Exec *e, const Dag &dag, int mode, const LowerOpts &lopts,
                             lane[u] = 0;
         // the kernel a unit's items run on: GEMM/SYRK blocks on k_batch_gemm,
         // small diagonal factorizations / conversions on k_batch_small, panel
-        // solves with inverted diagonal blocks (and the inversions, TRINV) on
-        // the 4-wave k_batch_trsm_mid<256 / 512> or, for larger triangles, the
-        // 8-wave k_batch_trsm, small solves without inverses on
-        // k_batch_trsm_small; anything else on the generic k_batch
+        // solves of order <= 128 / 256 on k_batch_trsm_small / k_batch_trsm_256,
+        // larger ones, with inverted diagonal blocks (and the inversions,
+        // TRINV), on the 4-wave k_batch_trsm_512 or the 8-wave k_batch_trsm;
+        // anything else on the generic k_batch
         auto ukind = [&](const UnitDesc &d) -> int {
             if (d.op == OP_GEMM && (d.flags & F_NARROW))
                 return LEVEL_GEMM_NARROW;
@@ -491,11 +491,11 @@ static int exec_build(Exec *e, const Dag &dag, int mode, const LowerOpts &lopts,
             if (small_only_op(d.op))
                 return LEVEL_SMALL;
             if (d.op == OP_TRINV)
-                return LEVEL_TRSM_256;
+                return LEVEL_TRSM_512;
             if (d.op == OP_TRSM && (d.flags & F_INV))
-                return d.m <= 256 ? LEVEL_TRSM_256 : d.m <= 512 ? LEVEL_TRSM_512 : LEVEL_TRSM;
-            if (d.op == OP_TRSM && d.m <= SMALL_MAX)
-                return LEVEL_TRSM_SMALL;
+                return d.m <= 512 ? LEVEL_TRSM_512 : LEVEL_TRSM;
+            if (d.op == OP_TRSM)
+                return d.m <= SMALL_MAX ? LEVEL_TRSM_SMALL : LEVEL_TRSM_256;
             return LEVEL_GENERIC;
         };
         // one kernel node per (level, lane, kernel) with work, in that order
@@ -648,8 +648,7 @@ static int exec_build(Exec *e, const Dag &dag, int mode, const LowerOpts &lopts,
     // bodies (the lowering options of this mode guarantee it)
     for (uint32_t u = 0; u < nu; u++) {
         const UnitDesc &d = L.units[u];
-        const bool ok = (d.op == OP_TRSM && (d.flags & F_INV)) ? d.m <= PERSIST_TRSM_MAX
-                        : d.op == OP_TRSM                      ? d.m <= SMALL_MAX
+        const bool ok = d.op == OP_TRSM ? d.m <= PERSIST_TRSM_MAX
                         : (d.op == OP_GETRF || d.op == OP_POTRF) ? d.m <= SMALL_MAX
                                                                  : true;
         if (!ok) {

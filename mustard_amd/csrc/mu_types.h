@@ -17,10 +17,11 @@ enum Op : int32_t {
     OP_NONE = 0,
     OP_GEMM = 1,   // C <- beta C + alpha op(A) op(B); items = bm x bn output blocks
     OP_SYRK = 2,   // lower(C) <- beta C + alpha A A^T; items = lower output blocks
-    OP_TRSM = 3,   // panel triangular solve T Y = Z; items = panels of <= 16 right-hand sides
+    OP_TRSM = 3,   // panel triangular solve T Y = Z; items = panels of <= 64 right-hand sides
+                   // (F_INV: <= 16)
     OP_GETRF = 4,  // no-pivot LU of an n <= SMALL_MAX tile in LDS; one item
     OP_POTRF = 5,  // lower Cholesky of an n <= SMALL_MAX tile in LDS; one item
-    OP_TRINV = 6,  // inverses of the 16 x 16 diagonal blocks of a TRSM triangle, into the
+    OP_TRINV = 6,  // inverses of the 16 x 16 diagonal blocks of an F_INV triangle, into the
                    // unit's workspace slot; items = groups of TRINV_BLOCKS blocks
     OP_CVT = 7,    // FP64 block (c, ldc) rounded to FP32 / BF16 storage (b, ldb); items = 64 x 64
 };
@@ -36,7 +37,8 @@ enum Flag : int32_t {
     F_LOW_F32 = 1 << 6,  // GEMM/SYRK: operands rounded to FP32, FP32 MFMA, FP32 accumulation
     F_LOW_BF16 = 1 << 7, // GEMM/SYRK: operands rounded to BF16, FP32 accumulation
     F_REV = 1 << 8,      // TRSM: row order of T and Z reversed (upper-triangular solves)
-    F_INV = 1 << 9,      // TRSM: diagonal blocks solved with the inverses a TRINV unit left in b
+    F_INV = 1 << 9,      // TRSM of order > TRSM_REG_MAX: diagonal blocks solved with the inverses
+                         // a TRINV unit left in b
     F_SRC_LOW = 1 << 10, // GEMM/SYRK with F_LOW_*: a and b are stored in that precision (not FP64)
     F_NARROW = 1 << 11,  // GEMM (FP64, op(B) = B) with n <= 16: items are 16-row tiles, every
                          // column in one item
@@ -60,7 +62,9 @@ constexpr int WG_THREADS = 256;
 constexpr int GEMM_BM = 64;     // GEMM/SYRK output block rows per item
 constexpr int GEMM_BN = 64;     // ... and columns
 constexpr int GEMM_BK = 8;      // k-block staged in LDS per step
-constexpr int TRSM_W = 16;        // right-hand sides per TRSM item
+constexpr int TRSM_W = 16;        // right-hand sides per wave (F_INV: per workgroup) of a TRSM item
+constexpr int TRSM_REG_MAX = 256; // largest triangle a TRSM item solves in registers, 4 * TRSM_W
+                                  // right-hand sides per item; larger ones (F_INV) in LDS
 constexpr int TRSM_NMAX = 1024;   // largest triangle a TRSM item keeps in LDS
 constexpr int TRSM_NEST = 256;    // default: triangles above this order nest into blocks,
                                   // whose solves run beside GEMM workgroups on a CU
