@@ -233,53 +233,81 @@ __global__ void k_fill_u64(unsigned long long *p, int n, unsigned long long v)
         p[i] = v;
 }
 
-// Residuals of a batch of packed problems, one workgroup per problem p of
-// order n = ns[p]: A_p (n x n, leading dimension n) at A + a_off[p], x_p, b_p
-// and r_p at v_off[p] of X, B and R.  r = b - A x in FP64, and the four
-// maxima of the LAPACK stopping test, ||r||_inf, ||x||_inf, ||A||_inf and
-// ||b||_inf, into norms[4p .. 4p+3].  A thread owns rows tid, tid + 256, ...
-// and walks them along the columns (a wave reads 64 consecutive rows of a
-// column); maxima on the bit patterns of non-negative values (a NaN's
-// pattern sorts above inf, so NaN propagates).
-__global__ __launch_bounds__(256) void k_batch_residual(const int *ns, const long long *a_off,
-                                                        const long long *v_off, const double *A,
-                                                        const double *X, const double *B,
-                                                        double *R, double *norms)
+// Residuals of a batch of packed problems p of order n = ns[p]: A_p (n x n,
+// leading dimension n) at A + a_off[p], x_p, b_p and r_p at v_off[p] of X, B
+// and R.  r = b - A x in FP64, and the four maxima of the LAPACK stopping
+// test, ||r||_inf, ||x||_inf, ||A||_inf and ||b||_inf, into norms[4p ..
+// 4p+3] (zeroed before).  Memory-bound: every element of A is read once.  A
+// workgroup takes 64 rows, its four waves every fourth group of 16 columns
+// (a wave reads 64 consecutive rows of a column, 16 loads in flight), and
+// BRES_WGS workgroups share a problem; with one workgroup per problem and a
+// thread per row, the largest problem's rows were one serial chain of n
+// loads (288 problems of order 32..1024: 1660 -> 103 us).  A row's four partial sums
+// are added in a fixed order.  Maxima on the bit patterns of non-negative
+// values (a NaN's pattern sorts above inf, so NaN propagates).
+constexpr int BRES_WGS = 16;
+
+__global__ __launch_bounds__(256) void k_batch_residual(
+    const int *__restrict__ ns, const long long *__restrict__ a_off,
+    const long long *__restrict__ v_off, const double *__restrict__ A,
+    const double *__restrict__ X, const double *__restrict__ B, double *__restrict__ R,
+    unsigned long long *norms)
 {
-    const int p = blockIdx.x, n = ns[p];
+    const int p = blockIdx.y, n = ns[p];
     const double *a = A + a_off[p];
     const double *x = X + v_off[p], *b = B + v_off[p];
     double *r = R + v_off[p];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    __shared__ double part[2][4][64];
     unsigned long long mr = 0, mx = 0, ma = 0, mb = 0;
     auto bits = [](double v) { return (unsigned long long)__double_as_longlong(fabs(v)); };
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    for (int r0 = blockIdx.x * 64; r0 < n; r0 += gridDim.x * 64) {
+        const int i = r0 + lane;
+        const double *ai = a + min(i, n - 1);
         double acc = 0.0, asum = 0.0;
-        for (int j = 0; j < n; j++) {
-            const double v = a[i + (size_t)j * n];
-            acc = fma(v, x[j], acc);
+        int j = 16 * w;
+        for (; j + 16 <= n; j += 64) {
+            double v[16];
+#pragma unroll
+            for (int q = 0; q < 16; q++)
+                v[q] = ai[(size_t)(j + q) * n];
+#pragma unroll
+            for (int q = 0; q < 16; q++) {
+                acc = fma(v[q], x[j + q], acc);
+                asum += fabs(v[q]);
+            }
+        }
+        for (int q = j; q < min(j + 16, n); q++) {
+            const double v = ai[(size_t)q * n];
+            acc = fma(v, x[q], acc);
             asum += fabs(v);
         }
-        const double ri = b[i] - acc;
-        r[i] = ri;
-        mr = max(mr, bits(ri));
-        mx = max(mx, bits(x[i]));
-        ma = max(ma, bits(asum));
-        mb = max(mb, bits(b[i]));
-    }
-    __shared__ unsigned long long red[4][256];
-    red[0][threadIdx.x] = mr;
-    red[1][threadIdx.x] = mx;
-    red[2][threadIdx.x] = ma;
-    red[3][threadIdx.x] = mb;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int q = 0; q < 4; q++)
-                red[q][threadIdx.x] = max(red[q][threadIdx.x], red[q][threadIdx.x + w]);
+        part[0][w][lane] = acc;
+        part[1][w][lane] = asum;
+        __syncthreads();
+        if (w == 0 && i < n) {
+            acc = (part[0][0][lane] + part[0][1][lane]) + (part[0][2][lane] + part[0][3][lane]);
+            asum = (part[1][0][lane] + part[1][1][lane]) + (part[1][2][lane] + part[1][3][lane]);
+            const double ri = b[i] - acc;
+            r[i] = ri;
+            mr = max(mr, bits(ri));
+            mx = max(mx, bits(x[i]));
+            ma = max(ma, bits(asum));
+            mb = max(mb, bits(b[i]));
+        }
         __syncthreads();
     }
-    if (threadIdx.x < 4)
-        norms[4 * p + threadIdx.x] = __longlong_as_double((long long)red[threadIdx.x][0]);
+    if (w != 0 || (int)blockIdx.x * 64 >= n)
+        return;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+        mr = max(mr, (unsigned long long)__shfl_xor((long long)mr, d));
+        mx = max(mx, (unsigned long long)__shfl_xor((long long)mx, d));
+        ma = max(ma, (unsigned long long)__shfl_xor((long long)ma, d));
+        mb = max(mb, (unsigned long long)__shfl_xor((long long)mb, d));
+    }
+    if (lane < 4)
+        atomicMax(norms + 4 * (size_t)p + lane, lane == 0 ? mr : lane == 1 ? mx : lane == 2 ? ma : mb);
 }
 
 int batch_residual(int nprob, const int *ns, const long long *a_off, const long long *v_off,
@@ -288,8 +316,15 @@ int batch_residual(int nprob, const int *ns, const long long *a_off, const long 
 {
     if (nprob <= 0)
         return 0;
-    hipLaunchKernelGGL(k_batch_residual, dim3(nprob), dim3(256), 0, s, ns, a_off, v_off, A, X, B,
-                       R, norms);
+    unsigned long long *nm = reinterpret_cast<unsigned long long *>(norms);
+    hipLaunchKernelGGL(k_fill_u64, dim3((4 * (unsigned)nprob + 255) / 256), dim3(256), 0, s, nm,
+                       4 * nprob, 0ull);
+    // grid.y holds at most 65535 problems
+    for (int p = 0; p < nprob; p += 65535) {
+        const int np = std::min(nprob - p, 65535);
+        hipLaunchKernelGGL(k_batch_residual, dim3(BRES_WGS, np), dim3(256), 0, s, ns + p, a_off + p,
+                           v_off + p, A, X, B, R, nm + 4 * (size_t)p);
+    }
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
