@@ -434,6 +434,10 @@ struct Builder {
                 UnitDesc d = base(op);
                 d.gm = 1;
                 d.gn = cdiv(op.n, 4 * TRSM_W);
+                // one item either way, and the four waves share it (launches of
+                // few wider panels are split where they are put together)
+                if (op.m <= TRSM_REG_MAX && op.n <= TRSM_W)
+                    d.flags |= F_SPLIT;
                 if (op.m > TRSM_REG_MAX) {
                     d.gn = cdiv(op.n, TRSM_W);
                     // the triangle's 16 x 16 diagonal blocks are inverted once,

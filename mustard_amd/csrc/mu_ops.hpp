@@ -2017,6 +2017,234 @@ __device__ __attribute__((always_inline)) inline void trsm_panel_reg(const UnitD
         }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // copies past the triangle have landed
 }
+
+// ---------------------------------------------------------------------------
+// The same solve with one panel of <= 16 right-hand sides on the whole
+// workgroup (units flagged F_SPLIT).
+//
+// What bounds it: the chain over the 16-row blocks.  trsm_panel_reg runs the
+// n / 16 (n / 16 + 1) / 2 block products of a panel one after another on one
+// wave (order 250: 39 us, 16 of them MFMA issue); here block row i belongs to
+// wave i % 4, so a step of the chain is X_j = inv(T_jj) Y_j on its owner, a
+// hand-over through LDS with one barrier, and the update of row j + 1; the
+// owner of row j + 1 puts off its other rows until X_{j+1} is out.  The
+// elements take the same updates in the same order, so the results are those
+// of trsm_panel_reg to the bit.  Order 250, one panel: 39 -> 19 us (8.5 us of
+// it the chain: 1400 cycles a step, 1000 where a wave has two rows), order 125
+// 14.5 -> 11 us; LU solve n = 12000, 16 right-hand sides, 5.17 -> 3.16 ms.
+//
+// T is read straight into the MFMA operand by the wave that uses it,
+// TRSM_SPLIT_AHEAD columns ahead.  Nothing but the two products, the LDS
+// traffic and one barrier is left on the chain: the inverses are in registers,
+// and a load's address is a scalar pointer per block row, moved on by one
+// scalar addition per column, plus a lane offset fixed for the whole solve
+// (with addresses computed block by block a step took 2000 cycles).  Three
+// columns ahead, or touching all of T first, measured the same or slower.
+// ---------------------------------------------------------------------------
+constexpr int TRSM_SPLIT_AHEAD = 2;  // columns of T in registers
+
+template <int NS>
+struct TrsmSplit {
+    // NS block rows per wave, row 4 k + wave in slot k; block rows nb - 1 ..
+    // 4 NS - 1 lie in the last slot
+    const MU_G char *t[NS];    // T's block (row of slot k, next column), its lowest address
+    unsigned tl[4], tlast[4];  // this lane's byte offset of element e, and in the last slot
+    long long step;            // bytes to the next column
+    int nb, wave;
+    v2d *xb;                   // this lane's part of -X_j, two buffers of 256 doubles
+    v4d Y[NS], W[NS], T[TRSM_SPLIT_AHEAD][NS];
+
+    // T's column j into d, slots K0 .. (slots above the diagonal read the
+    // other triangle and are never used); then on to column j + 1, which
+    // stops at the last column with blocks below it
+    template <int K0>
+    __device__ __forceinline__ void load(v4d (&d)[NS], int j)
+    {
+        const long long s = j < nb - 2 ? step : 0;
+#pragma unroll
+        for (int k = 0; k < NS; k++) {
+            if (k >= K0)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    d[k][e] = *(const MU_G double *)(t[k] + (k == NS - 1 ? tlast[e] : tl[e]));
+            t[k] += s;
+        }
+    }
+    __device__ __forceinline__ void update(v4d &y, const v4d &tb, const v4d &nx)
+    {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            y = mfma_f64(tb[e], nx[e], y);
+    }
+    // X_J on its owner; rows past n (rlast as in trsm_columns) are zero before
+    template <int J>
+    __device__ __forceinline__ void solve(int rlast)
+    {
+        v4d &y = Y[J / 4];
+        if (J / 4 == NS - 1 && J == nb - 1)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                y[e] = 4 * e < rlast ? y[e] : 0.0;
+        v4d x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            x = mfma_f64(W[J / 4][e], y[e], x);
+        y = x;
+        v2d *o = xb + (J & 1) * 128;
+        o[0] = v2d{-x[0], -x[1]};
+        o[64] = v2d{-x[2], -x[3]};
+    }
+    // the barrier, with the MFMAs kept on their side of it
+    static __device__ __forceinline__ void barrier()
+    {
+        __builtin_amdgcn_sched_barrier(0);
+        lds_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // Steps J ..: every wave sees X_J in its buffer.
+    template <int J>
+    __device__ __forceinline__ void steps(int rlast)
+    {
+        if constexpr (J + 1 < 4 * NS) {
+            if (J + 1 >= nb)
+                return;
+            // row J + 1: slot S of wave w
+            constexpr int S = (J + 1) / 4, w = (J + 1) & 3, B = J % TRSM_SPLIT_AHEAD;
+            const v2d n0 = xb[(J & 1) * 128], n1 = xb[(J & 1) * 128 + 64];
+            const v4d nx = {n0[0], n0[1], n1[0], n1[1]};
+            if (wave == w) {
+                update(Y[S], T[B][S], nx);
+                __builtin_amdgcn_sched_barrier(0);
+                solve<J + 1>(rlast);
+                barrier();
+#pragma unroll
+                for (int k = S + 1; k < NS; k++)
+                    update(Y[k], T[B][k], nx);
+            } else {
+                if (wave > w)
+                    update(Y[S], T[B][S], nx);
+#pragma unroll
+                for (int k = S + 1; k < NS; k++)
+                    update(Y[k], T[B][k], nx);
+                barrier();
+            }
+            if constexpr (J + TRSM_SPLIT_AHEAD < 4 * NS - 1)
+                load<(J + TRSM_SPLIT_AHEAD + 1) / 4>(T[B], J + TRSM_SPLIT_AHEAD);
+            steps<J + 1>(rlast);
+        }
+    }
+};
+
+template <int NS>
+__device__ __attribute__((always_inline)) inline void trsm_panel_split(const UnitDesc &u, int it,
+                                                                       double *smem)
+{
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = __builtin_amdgcn_readfirstlane(u.m), nb = (n + 15) >> 4;
+    const int ncol = __builtin_amdgcn_readfirstlane(u.n);
+    const int flags = __builtin_amdgcn_readfirstlane(u.flags);
+    const bool rev = flags & F_REV, tt = flags & F_T_TRANS, zr = flags & F_Z_ROWS;
+    const unsigned ldt = __builtin_amdgcn_readfirstlane(u.lda);
+    const unsigned ldz = __builtin_amdgcn_readfirstlane(u.ldc);
+    const MU_G double *t = gp(uniform_ptr(u.a));
+    MU_G double *z = gp(uniform_ptr(u.c));
+    const double alpha = u.alpha;
+    const int nlast = n - 16 * (nb - 1);
+    const unsigned rs = tt ? ldt : 1, cs = tt ? 1 : ldt;
+    const unsigned zrs = zr ? ldz : 1, zcs = zr ? 1 : ldz;
+
+    TrsmSplit<NS> p;
+    p.nb = nb;
+    p.wave = wave;
+    p.xb = reinterpret_cast<v2d *>(smem + 4 * NS * BF_BLK) + lane;
+
+    // ---- the diagonal blocks, block wave + 4 lk on this group
+    const int jb = min(wave + 4 * lk, nb - 1), r = 16 * jb + li, rc = min(r, n - 1);
+    double x[16], v[16];
+    {
+        // rows past n: the last one; columns past n: the last one
+        const size_t a = (size_t)(rev ? n - 1 - rc : rc) * rs;
+#pragma unroll
+        for (int c = 0; c < 16; c++) {
+            const int cc = min(16 * jb + c, n - 1);
+            x[c] = t[a + (size_t)(rev ? n - 1 - cc : cc) * cs];
+        }
+    }
+    const double dv = t[(size_t)(rev ? n - 1 - rc : rc) * (rs + (size_t)cs)];
+
+    // ---- the panel (rows past n: the last one)
+    const int p0 = it * TRSM_W, w = min(TRSM_W, ncol - p0), lic = min(li, w - 1);
+    MU_G double *zb = z + (size_t)p0 * zcs;
+    auto zat = [&](int row) -> MU_G double * {
+        return zb + ((size_t)(rev ? n - 1 - row : row) * zrs + (size_t)lic * zcs);
+    };
+#pragma unroll
+    for (int k = 0; k < NS; k++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            p.Y[k][e] = *zat(min(16 * (4 * k + wave) + 4 * e + lk, n - 1));
+
+    // ---- T's first columns.  With rev a block lies mirrored; in the last
+    // block row the rows past n are the last one.
+    if (nb > 1) {
+        p.step = (rev ? -128 : 128) * (long long)cs;
+#pragma unroll
+        for (int k = 0; k < NS; k++) {
+            const int i = min(4 * k + wave, nb - 1);
+            p.t[k] = (const MU_G char *)(t + (size_t)(rev ? max(n - 16 - 16 * i, 0) : 16 * i) * rs +
+                                         (size_t)(rev ? n - 16 : 0) * cs);
+        }
+        const bool last = 4 * (NS - 1) + wave >= nb - 1;
+        const unsigned ro = rev ? 15 - li : li;
+        const unsigned rl = last ? (rev ? max(nlast - 1 - li, 0) : min(li, nlast - 1)) : ro;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const unsigned c = rev ? 15 - 4 * e - lk : 4 * e + lk;
+            p.tl[e] = 8 * (ro * rs + c * cs);
+            p.tlast[e] = 8 * (rl * rs + c * cs);
+        }
+#pragma unroll
+        for (int j = 0; j < TRSM_SPLIT_AHEAD; j++)
+            p.template load<0>(p.T[j], j);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    // ---- the inverses; a wave reads back those of its own rows
+#pragma unroll
+    for (int c = 0; c < 16; c++) {
+        x[c] = r < n ? x[c] : 0.0;
+        v[c] = c == li ? 1.0 : 0.0;
+    }
+    const double rd = ((flags & F_UNIT) || r >= n) ? 1.0 : 1.0 / dv;
+    tri_inv16<0>(v, x, rd, smem + jb * BF_BLK + li);
+    lds_barrier();  // the last block's inverse may have been formed by every wave
+#pragma unroll
+    for (int k = 0; k < NS; k++) {
+        const double *b = smem + min(4 * k + wave, nb - 1) * BF_BLK + li * BF_LD + lk;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            p.W[k][e] = b[4 * e];
+            p.Y[k][e] *= alpha;
+        }
+    }
+
+    if (wave == 0)
+        p.template solve<0>(nlast - lk);
+    p.barrier();
+    p.template steps<0>(nlast - lk);
+
+    if (li < w)
+#pragma unroll
+        for (int k = 0; k < NS; k++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int row = 16 * (4 * k + wave) + 4 * e + lk;
+                if (row < n)
+                    *zat(row) = p.Y[k][e];
+            }
+}
+
 constexpr int LDS_TRSM_REG = 16 * BF_BLK + TRSM_RING<16> * 1024;       // inverses of order TRSM_REG_MAX
 constexpr int LDS_TRSM_REG_SMALL = 8 * BF_BLK + TRSM_RING<8> * 1024;  // ... of order SMALL_MAX
 
@@ -2028,6 +2256,17 @@ __device__ __attribute__((always_inline)) inline void run_trsm_reg_item(const Un
                                                                         double *smem)
 {
     const int nb = (__builtin_amdgcn_readfirstlane(u.m) + 15) >> 4;
+    if (__builtin_amdgcn_readfirstlane(u.flags) & F_SPLIT) {
+        if (nb <= 4)
+            trsm_panel_split<1>(u, it, smem);
+        else if (MAXNB == 8 || nb <= 8)
+            trsm_panel_split<2>(u, it, smem);
+        else if (nb <= 12)
+            trsm_panel_split<MAXNB == 8 ? 2 : 3>(u, it, smem);
+        else
+            trsm_panel_split<MAXNB == 8 ? 2 : 4>(u, it, smem);
+        return;
+    }
     if (nb <= 2)
         trsm_panel_reg<2>(u, it, smem);
     else if (nb <= 4)

@@ -266,6 +266,27 @@ static std::vector<uint32_t> merge_node(const std::vector<UnitDesc> &lowered,
     return out;
 }
 
+// Panel solves of a launch with fewer items than this run on panels of 16
+// right-hand sides, four waves each (F_SPLIT), instead of 64.  Such a panel
+// takes half the time, but its inverses are formed for 16 right-hand sides
+// instead of 64 and its waves wait for each other, so where 64-wide panels
+// fill the 256 CUs they win: limit 0 / 64 / 256 / 512, Cholesky 7007 5.91 /
+// 5.32 / 5.13 / 5.18 ms, LU 24000 153.3 / 152.9 / 153.0 / 154.1 ms; split
+// whatever the count, LU 24000 159 ms and the batch of 4608 10.8 -> 12.4 ms.
+constexpr int TRSM_SPLIT_ITEMS = 256;
+
+static bool can_split(const UnitDesc &d, int launch_items)
+{
+    return d.op == OP_TRSM && !(d.flags & (F_INV | F_SPLIT)) && launch_items < TRSM_SPLIT_ITEMS;
+}
+static UnitDesc split_panels(UnitDesc d)
+{
+    d.flags |= F_SPLIT;
+    d.gn = (d.n + TRSM_W - 1) / TRSM_W;
+    d.nitems = unit_items(d);
+    return d;
+}
+
 int run_units(const Lowered &low, hipStream_t s, std::string &err)
 {
     // units of an executable come patched; an eager call gets a
@@ -300,7 +321,7 @@ int run_units(const Lowered &low, hipStream_t s, std::string &err)
     for (const UnitDesc &d : low.units) {
         if (d.nitems <= 0)
             continue;
-        if (launch_unit(d, s) != 0)
+        if (launch_unit(can_split(d, d.nitems) ? split_panels(d) : d, s) != 0)
             HIPCHK(hipGetLastError());
     }
     return 0;
@@ -534,6 +555,14 @@ static int exec_build(Exec *e, const Dag &dag, int mode, const LowerOpts &lopts,
                             d.gn = d.op == OP_SYRK ? d.gm : (d.n + 127) / 128;
                             u = mo.add(d);
                         }
+                    if (k % NK == LEVEL_TRSM_SMALL || k % NK == LEVEL_TRSM_256) {
+                        int ni = 0;
+                        for (uint32_t u : us)
+                            ni += e->gunits[u].nitems;
+                        for (uint32_t &u : us)
+                            if (can_split(e->gunits[u], ni))
+                                u = mo.add(split_panels(e->gunits[u]));
+                    }
                     std::vector<uint32_t> its;
                     for (uint32_t u : us)
                         for (int i = 0; i < e->gunits[u].nitems; i++)

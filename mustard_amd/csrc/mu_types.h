@@ -18,7 +18,7 @@ enum Op : int32_t {
     OP_GEMM = 1,   // C <- beta C + alpha op(A) op(B); items = bm x bn output blocks
     OP_SYRK = 2,   // lower(C) <- beta C + alpha A A^T; items = lower output blocks
     OP_TRSM = 3,   // panel triangular solve T Y = Z; items = panels of <= 64 right-hand sides
-                   // (F_INV: <= 16)
+                   // (F_INV, F_SPLIT: <= 16)
     OP_GETRF = 4,  // no-pivot LU of an n <= SMALL_MAX tile in LDS; one item
     OP_POTRF = 5,  // lower Cholesky of an n <= SMALL_MAX tile in LDS; one item
     OP_TRINV = 6,  // inverses of the 16 x 16 diagonal blocks of an F_INV triangle, into the
@@ -55,6 +55,8 @@ enum Flag : int32_t {
     F_CVT_BOTH = 1 << 16, // CVT with F_CVT_T: also stores the block untransposed at (a, lda)
     F_BROW = 1 << 17,    // F_A32 GEMM: B and C stored by rows (B(k, j) at b[k*ldb + j], C(i, j)
                          // at c[i*ldc + j])
+    F_SPLIT = 1 << 18,   // TRSM without F_INV: items are panels of <= 16 right-hand sides, each on
+                         // all four waves
 };
 
 // Kernel geometry (fixed for gfx950: 4 waves of 64 lanes per workgroup).
