@@ -624,6 +624,7 @@ int mu_exec_create(mu_dag_t dag, int mode, const mu_exec_opts_t *opts, mu_exec_t
     if (mode == MU_MODE_SUBGRAPH) {
         lo.trsm_max = std::min(lo.trsm_max, mu::PERSIST_TRSM_MAX);
         lo.gemm_group = 2;
+        lo.nest_panels = false;
     }
     for (const auto &t : dag->dag.tasks)
         for (const auto &op : t.ops)
@@ -795,6 +796,7 @@ static int emulate_into(mu_dag_t dag, const mu::EmuOpts &eo, long long *results,
     mu::LowerOpts lo;
     lo.trsm_max = std::min(lo.trsm_max, mu::PERSIST_TRSM_MAX);
     lo.gemm_group = 2;
+    lo.nest_panels = false;
     if (!mu::emulate(dag->dag, lo, eo, r, err))
         return fail(MU_EINVAL, err);
     const long long v[9] = {(long long)r.executed, (long long)r.duplicates,

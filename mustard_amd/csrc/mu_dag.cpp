@@ -497,6 +497,9 @@ struct Builder {
         auto blk = [&](int i, int j) { return op.c + bd[i] + (size_t)bd[j] * ld; };
         auto sz = [&](int i) { return bd[i + 1] - bd[i]; };
         SubRec rec(*this);
+        // one panel instead of P - 1 - k blocks of it, where nothing waits
+        // for a single block
+        const bool whole = o.nest_panels && !outer;
         for (int k = 0; k < P; k++) {
             OpRec g;
             g.op = OP_GETRF;
@@ -507,12 +510,14 @@ struct Builder {
             g.info_base = op.info_base + bd[k];
             if (!rec.add({k, k}, {{k, k}}, g))
                 return false;
-            for (int i = k + 1; i < P; i++) {
+            auto cols = [&](int i) { return whole ? n - bd[i] : sz(i); };
+            const int end = whole ? std::min(k + 2, P) : P;
+            for (int i = k + 1; i < end; i++) {
                 OpRec t;
                 t.op = OP_TRSM;
                 t.flags = F_UNIT;
                 t.m = sz(k);
-                t.n = sz(i);
+                t.n = cols(i);
                 t.a = blk(k, k);
                 t.lda = (int)ld;
                 t.c = blk(k, i);
@@ -521,12 +526,12 @@ struct Builder {
                 if (!rec.add({k, i}, {{k, k}, {k, i}}, t, {k, k}))
                     return false;
             }
-            for (int i = k + 1; i < P; i++) {
+            for (int i = k + 1; i < end; i++) {
                 OpRec t;
                 t.op = OP_TRSM;
                 t.flags = F_T_TRANS | F_Z_ROWS;
                 t.m = sz(k);
-                t.n = sz(i);
+                t.n = cols(i);
                 t.a = blk(k, k);
                 t.lda = (int)ld;
                 t.c = blk(i, k);
@@ -534,11 +539,11 @@ struct Builder {
                 t.alpha = 1.0;
                 if (!rec.add({i, k}, {{k, k}, {i, k}}, t, {k, k}))
                     return false;
-                for (int j = k + 1; j < P; j++) {
+                for (int j = k + 1; j < end; j++) {
                     OpRec g2;
                     g2.op = OP_GEMM;
-                    g2.m = sz(i);
-                    g2.n = sz(j);
+                    g2.m = cols(i);
+                    g2.n = cols(j);
                     g2.k = sz(k);
                     g2.a = blk(i, k);
                     g2.lda = (int)ld;
@@ -568,6 +573,7 @@ struct Builder {
         auto blk = [&](int i, int j) { return op.c + bd[i] + (size_t)bd[j] * ld; };
         auto sz = [&](int i) { return bd[i + 1] - bd[i]; };
         SubRec rec(*this);
+        const bool whole = o.nest_panels && !outer;  // as in lower_getrf_nested
         for (int k = 0; k < P; k++) {
             OpRec p;
             p.op = OP_POTRF;
@@ -578,12 +584,14 @@ struct Builder {
             p.info_base = op.info_base + bd[k];
             if (!rec.add({k, k}, {{k, k}}, p))
                 return false;
-            for (int i = k + 1; i < P; i++) {
+            auto rows = [&](int i) { return whole ? n - bd[i] : sz(i); };
+            const int end = whole ? std::min(k + 2, P) : P;
+            for (int i = k + 1; i < end; i++) {
                 OpRec t;
                 t.op = OP_TRSM;
                 t.flags = F_Z_ROWS;
                 t.m = sz(k);
-                t.n = sz(i);
+                t.n = rows(i);
                 t.a = blk(k, k);
                 t.lda = (int)ld;
                 t.c = blk(i, k);
@@ -592,10 +600,10 @@ struct Builder {
                 if (!rec.add({i, k}, {{k, k}, {i, k}}, t, {k, k}))
                     return false;
             }
-            for (int i = k + 1; i < P; i++) {
+            for (int i = k + 1; i < end; i++) {
                 OpRec s;
                 s.op = OP_SYRK;
-                s.n = s.m = sz(i);
+                s.n = s.m = rows(i);
                 s.k = sz(k);
                 s.a = blk(i, k);
                 s.lda = (int)ld;
@@ -605,7 +613,7 @@ struct Builder {
                 s.update = outer;
                 if (!rec.add({i, i}, {{i, i}, {i, k}}, s))
                     return false;
-                for (int j = i + 1; j < P; j++) {
+                for (int j = i + 1; j < end; j++) {
                     OpRec g;
                     g.op = OP_GEMM;
                     g.flags = F_TB | (op.flags & (F_LOW_F32 | F_LOW_BF16));

@@ -82,6 +82,14 @@ struct LowerOpts {
     // so a whole-matrix task lowers like the tiled DAG instead of into
     // (n / small_max)^2 sub-tiles.
     int nest_outer = 1000;
+    // A factorization nested in one level: one panel solve and one update
+    // over everything below (and right of) a diagonal block, instead of one
+    // per pair of blocks.  The level-batched graph runs the parts of a step
+    // as one node anyway, and blocks of 65..127 cost the GEMM 64-row blocks
+    // that overlap (a 70 x 70 update runs as 128 x 128).  Off for the
+    // persistent scheduler, whose next diagonal block starts after its own
+    // update alone.
+    bool nest_panels = true;
 };
 
 struct Lowered {
