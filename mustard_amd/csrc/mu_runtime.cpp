@@ -287,6 +287,37 @@ static UnitDesc split_panels(UnitDesc d)
     return d;
 }
 
+// The items of a node in launch order.  Workgroup p runs on XCD p % 8, each
+// with an L2 of its own, and the items of a unit share operands.  In a node of
+// many units (a batch: one or a few per problem) every unit is given to one
+// XCD, the one with the fewest items so far; one after the other they would
+// spread a problem's items over all eight, and each would read its panels
+// from memory.
+constexpr size_t XCDS = 8, XCD_UNITS = 64;
+
+static std::vector<uint32_t> node_items(const std::vector<UnitDesc> &units,
+                                        const std::vector<uint32_t> &ids)
+{
+    const size_t nq = ids.size() < XCD_UNITS ? 1 : XCDS;
+    std::vector<std::vector<uint32_t>> q(nq);
+    size_t total = 0;
+    for (uint32_t u : ids) {
+        auto &l = *std::min_element(q.begin(), q.end(), [](const auto &x, const auto &y) {
+            return x.size() < y.size();
+        });
+        for (int i = 0; i < units[u].nitems; i++)
+            l.push_back(units[u].item_base + i);
+        total += (size_t)units[u].nitems;
+    }
+    std::vector<uint32_t> out;
+    out.reserve(total);
+    for (size_t i = 0; out.size() < total; i++)
+        for (auto &l : q)
+            if (i < l.size())
+                out.push_back(l[i]);
+    return out;
+}
+
 int run_units(const Lowered &low, hipStream_t s, std::string &err)
 {
     // units of an executable come patched; an eager call gets a
@@ -563,10 +594,7 @@ static int exec_build(Exec *e, const Dag &dag, int mode, const LowerOpts &lopts,
                             if (can_split(e->gunits[u], ni))
                                 u = mo.add(split_panels(e->gunits[u]));
                     }
-                    std::vector<uint32_t> its;
-                    for (uint32_t u : us)
-                        for (int i = 0; i < e->gunits[u].nitems; i++)
-                            its.push_back(e->gunits[u].item_base + i);
+                    std::vector<uint32_t> its = node_items(e->gunits, us);
                     node_of[k] = (int)lv.size();
                     node_lane.push_back((int)((k / NK) % NL));
                     node_level.push_back((int)(k / NK / NL));
