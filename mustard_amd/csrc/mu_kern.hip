@@ -16,15 +16,14 @@ __global__ MU_GEMM_KERNEL void k_unit_gemm(UnitDesc d)
     run_gemm_item(d, blockIdx.x, smem);
 }
 
-__global__ MU_GEMM_KERNEL void k_batch_gemm(const UnitDesc *units, const uint32_t *item_unit,
-                                            const uint32_t *items)
+__global__ MU_GEMM_KERNEL void k_batch_gemm(NodeArgs node)
 {
     __shared__ __align__(16) double smem[LDS_GEMM];
-    const uint32_t item = items[blockIdx.x];
+    int it;
     // a private copy of the descriptor lives in registers; a reference into
     // global memory would be re-read after every barrier of the item body
-    const UnitDesc d = units[item_unit[item]];
-    run_gemm_item(d, (int)(item - d.item_base), smem);
+    const UnitDesc d = node_unit(node, it);
+    run_gemm_item(d, it, smem);
 }
 
 // Diagonal GETRF/POTRF (and precision conversions), 4 waves held to 200
@@ -33,12 +32,12 @@ __global__ MU_GEMM_KERNEL void k_batch_gemm(const UnitDesc *units, const uint32_
 // the diagonal factorization of the next step starts as soon as one bulk GEMM
 // workgroup leaves a CU instead of waiting for the bulk update to drain.
 __global__ __launch_bounds__(WG_THREADS) __attribute__((amdgpu_num_vgpr(100))) void
-k_batch_small(const UnitDesc *units, const uint32_t *item_unit, const uint32_t *items)
+k_batch_small(NodeArgs node)
 {
     __shared__ double smem[LDS_SMALL];
-    const uint32_t item = items[blockIdx.x];
-    const UnitDesc d = units[item_unit[item]];
-    run_small_item(d, (int)(item - d.item_base), smem);
+    int it;
+    const UnitDesc d = node_unit(node, it);
+    run_small_item(d, it, smem);
 }
 
 // Reduced-precision GEMM/SYRK units whose operands are k-contiguous in
@@ -46,73 +45,67 @@ k_batch_small(const UnitDesc *units, const uint32_t *item_unit, const uint32_t *
 // factorization reading the converted panels): long k-slices; 128 x 128
 // blocks in the level-batched graph (72 KB of LDS, two workgroups per CU).
 __global__ __launch_bounds__(WG_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void
-k_batch_gemm_low(const UnitDesc *units, const uint32_t *item_unit, const uint32_t *items)
+k_batch_gemm_low(NodeArgs node)
 {
     __shared__ double smem[LDS_GEMM_LOWK128];
-    const uint32_t item = items[blockIdx.x];
-    const UnitDesc d = units[item_unit[item]];
-    run_gemm_lowk_item(d, (int)(item - d.item_base), smem);
+    int it;
+    const UnitDesc d = node_unit(node, it);
+    run_gemm_lowk_item(d, it, smem);
 }
 
 // Precision conversions (the panels' reduced-precision shadows, the FP32
 // copies of the factors): 16 KB of LDS and few registers, so eight
 // workgroups share a CU -- a conversion on the lookahead chain waits for no
 // CU to drain, and the bulk ones stream at full occupancy.
-__global__ __launch_bounds__(WG_THREADS) void k_batch_cvt(const UnitDesc *units,
-                                                          const uint32_t *item_unit,
-                                                          const uint32_t *items)
+__global__ __launch_bounds__(WG_THREADS) void k_batch_cvt(NodeArgs node)
 {
     __shared__ double smem[4 * 16 * 65 / 2 + 4];
-    const uint32_t item = items[blockIdx.x];
-    const UnitDesc d = units[item_unit[item]];
-    cvt_block(d, (int)(item - d.item_base), smem);
+    int it;
+    const UnitDesc d = node_unit(node, it);
+    cvt_block(d, it, smem);
 }
 
 // GEMMs with at most 16 output columns (substitution steps of a solve).
-__global__ __launch_bounds__(WG_THREADS) void k_batch_gemm_narrow(const UnitDesc *units,
-                                                                  const uint32_t *item_unit,
-                                                                  const uint32_t *items)
+__global__ __launch_bounds__(WG_THREADS) void k_batch_gemm_narrow(NodeArgs node)
 {
     __shared__ double smem[LDS_NARROW];
-    const uint32_t item = items[blockIdx.x];
-    const UnitDesc d = units[item_unit[item]];
-    run_gemm_narrow_item(d, (int)(item - d.item_base), smem);
+    int it;
+    const UnitDesc d = node_unit(node, it);
+    run_gemm_narrow_item(d, it, smem);
 }
 
 // Panel solves of order <= SMALL_MAX (inside nested diagonal factorizations)
 // and of order <= TRSM_REG_MAX, at most 200 registers per lane as
 // k_batch_small, so they start beside three GEMM workgroups.
 __global__ __launch_bounds__(WG_THREADS) __attribute__((amdgpu_num_vgpr(100))) void
-k_batch_trsm_small(const UnitDesc *units, const uint32_t *item_unit, const uint32_t *items)
+k_batch_trsm_small(NodeArgs node)
 {
     __shared__ __align__(16) double smem[LDS_TRSM_REG_SMALL];
-    const uint32_t item = items[blockIdx.x];
-    const UnitDesc d = units[item_unit[item]];
-    run_trsm_reg_item<8>(d, (int)(item - d.item_base), smem);
+    int it;
+    const UnitDesc d = node_unit(node, it);
+    run_trsm_reg_item<8>(d, it, smem);
 }
 
 __global__ __launch_bounds__(WG_THREADS) __attribute__((amdgpu_num_vgpr(100))) void
-k_batch_trsm_256(const UnitDesc *units, const uint32_t *item_unit, const uint32_t *items)
+k_batch_trsm_256(NodeArgs node)
 {
     __shared__ __align__(16) double smem[LDS_TRSM_REG];
-    const uint32_t item = items[blockIdx.x];
-    const UnitDesc d = units[item_unit[item]];
-    run_trsm_reg_item<16>(d, (int)(item - d.item_base), smem);
+    int it;
+    const UnitDesc d = node_unit(node, it);
+    run_trsm_reg_item<16>(d, it, smem);
 }
 
 // Panel solves with inverted diagonal blocks of order <= 512, and the TRINV
 // items before them, on 4 waves and 64 KB of LDS (trsm_max above 256 only).
-__global__ __launch_bounds__(WG_THREADS) void k_batch_trsm_512(const UnitDesc *units,
-                                                               const uint32_t *item_unit,
-                                                               const uint32_t *items)
+__global__ __launch_bounds__(WG_THREADS) void k_batch_trsm_512(NodeArgs node)
 {
     __shared__ double smem[512 * 16];
-    const uint32_t item = items[blockIdx.x];
-    const UnitDesc d = units[item_unit[item]];
+    int it;
+    const UnitDesc d = node_unit(node, it);
     if (d.op == OP_TRINV)
-        run_trinv_item(d, (int)(item - d.item_base), smem);
+        run_trinv_item(d, it, smem);
     else
-        run_trsm_inv_item<4, 512>(d, (int)(item - d.item_base), smem);
+        run_trsm_inv_item<4, 512>(d, it, smem);
 }
 
 const void *level_kernel(int kind)

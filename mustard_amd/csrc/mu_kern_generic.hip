@@ -16,26 +16,22 @@ __global__ __launch_bounds__(WG_THREADS) void k_unit(UnitDesc d)
 }
 
 // One launch runs every item of one graph node; block b runs items[b].
-__global__ __launch_bounds__(WG_THREADS) void k_batch(const UnitDesc *units,
-                                                      const uint32_t *item_unit,
-                                                      const uint32_t *items)
+__global__ __launch_bounds__(WG_THREADS) void k_batch(NodeArgs node)
 {
     __shared__ __align__(16) double smem[LDS_DOUBLES];
-    const uint32_t item = items[blockIdx.x];
+    int it;
     // a private copy of the descriptor lives in registers; a reference into
     // global memory would be re-read after every barrier of the item body
-    const UnitDesc d = units[item_unit[item]];
-    run_item(d, (int)(item - d.item_base), smem);
+    const UnitDesc d = node_unit(node, it);
+    run_item(d, it, smem);
 }
 
-__global__ __launch_bounds__(64 * TRSM_KERNEL_WAVES) void k_batch_trsm(const UnitDesc *units,
-                                                                      const uint32_t *item_unit,
-                                                                      const uint32_t *items)
+__global__ __launch_bounds__(64 * TRSM_KERNEL_WAVES) void k_batch_trsm(NodeArgs node)
 {
     __shared__ double smem[TRSM_NMAX * 16];
-    const uint32_t item = items[blockIdx.x];
-    const UnitDesc d = units[item_unit[item]];
-    run_trsm_inv_item<TRSM_KERNEL_WAVES>(d, (int)(item - d.item_base), smem);
+    int it;
+    const UnitDesc d = node_unit(node, it);
+    run_trsm_inv_item<TRSM_KERNEL_WAVES>(d, it, smem);
 }
 
 const void *generic_kernel(int kind)

@@ -26,6 +26,7 @@ typedef double v2d __attribute__((ext_vector_type(2)));
 // infer their address space; they always point to device global memory, and
 // saying so turns flat accesses into global (vector memory) instructions.
 #define MU_G __attribute__((address_space(1)))
+#define MU_C __attribute__((address_space(4)))  // ... that no kernel writes meanwhile
 template <class T>
 __device__ __forceinline__ MU_G T *gp(T *p)
 {
@@ -2853,6 +2854,31 @@ __device__ __attribute__((always_inline)) inline void run_small_item(const UnitD
         potrf_small(u, smem);
     else
         cvt_block(u, it, smem);
+}
+
+// This workgroup's unit and item of a graph node.  The table's pointers come
+// in a structure, where the compiler does not see that they point to global
+// memory nothing writes: said here, the descriptor stays in scalar registers
+// (as flat loads it took 20 vector registers of every kernel).
+__device__ __forceinline__ UnitDesc node_unit(const NodeArgs &node, int &it)
+{
+    typedef unsigned v4u __attribute__((ext_vector_type(4)));
+    typedef unsigned v2u __attribute__((ext_vector_type(2)));
+    struct Words {
+        v4u w[sizeof(UnitDesc) / 16];
+    } w;
+    static_assert(sizeof(NodeItem) == sizeof(v2u) && sizeof(Words) == sizeof(UnitDesc), "");
+    if (!node.items) {
+        it = (int)blockIdx.x;
+        return node.one;
+    }
+    const v2u r = ((const MU_C v2u *)node.items)[blockIdx.x];
+    it = (int)r[1];
+    const MU_C v4u *p = (const MU_C v4u *)(node.units + r[0]);
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(UnitDesc) / 16); i++)
+        w.w[i] = p[i];
+    return __builtin_bit_cast(UnitDesc, w);
 }
 
 // Execute local item `it` of unit `u`.  Always inlined, so that LDS stays

@@ -646,22 +646,29 @@ static int exec_build(Exec *e, const Dag &dag, int mode, const LowerOpts &lopts,
             return r;
         };
         const size_t o_units = take(sizeof(UnitDesc) * std::max<uint32_t>(ngu, 1));
-        const size_t o_iu = take(sizeof(uint32_t) * std::max<size_t>(next_item, 1));
-        const size_t o_items = take(sizeof(uint32_t) * std::max<size_t>(items.size(), 1));
+        const size_t o_items = take(sizeof(NodeItem) * std::max<size_t>(items.size(), 1));
         e->dbytes = o;
         HIPCHK(hipMalloc(&e->dbuf, e->dbytes));
         if (ngu)
             HIPCHK(hipMemcpy(e->dbuf + o_units, e->gunits.data(), sizeof(UnitDesc) * ngu,
                              hipMemcpyHostToDevice));
-        if (next_item)
-            HIPCHK(hipMemcpy(e->dbuf + o_iu, item_unit.data(), sizeof(uint32_t) * next_item,
-                             hipMemcpyHostToDevice));
+        std::vector<NodeItem> nitems(items.size());
+        for (size_t i = 0; i < items.size(); i++) {
+            const uint32_t u = item_unit[items[i]];
+            nitems[i] = {u, items[i] - e->gunits[u].item_base};
+        }
         if (!items.empty())
-            HIPCHK(hipMemcpy(e->dbuf + o_items, items.data(), sizeof(uint32_t) * items.size(),
+            HIPCHK(hipMemcpy(e->dbuf + o_items, nitems.data(), sizeof(NodeItem) * nitems.size(),
                              hipMemcpyHostToDevice));
         const UnitDesc *du = reinterpret_cast<const UnitDesc *>(e->dbuf + o_units);
-        const uint32_t *diu = reinterpret_cast<const uint32_t *>(e->dbuf + o_iu);
-        const uint32_t *ditems = reinterpret_cast<const uint32_t *>(e->dbuf + o_items);
+        const NodeItem *ditems = reinterpret_cast<const NodeItem *>(e->dbuf + o_items);
+        e->level_args.resize(nnode);
+        for (int l = 0; l < nnode; l++) {
+            const NodeItem *ni = nitems.data() + off[l];
+            const UnitDesc &d = e->gunits[ni->unit];
+            const bool one = (size_t)d.nitems == lv[l].size() && ni[lv[l].size() - 1].unit == ni->unit;
+            e->level_args[l] = {du, one ? nullptr : ditems + off[l], d};
+        }
         e->level_flops.assign(nnode, 0.0);
         for (uint32_t u = 0; u < nu; u++)
             if (L.units[u].nitems > 0)
@@ -669,8 +676,7 @@ static int exec_build(Exec *e, const Dag &dag, int mode, const LowerOpts &lopts,
         HIPCHK(hipGraphCreate(&e->graph, 0));
         std::vector<hipGraphNode_t> gnodes(nnode);
         for (int l = 0; l < nnode; l++) {
-            const uint32_t *first = ditems + off[l];
-            void *args[] = {(void *)&du, (void *)&diu, (void *)&first};
+            void *args[] = {(void *)&e->level_args[l]};
             hipKernelNodeParams kp;
             std::memset(&kp, 0, sizeof kp);
             kp.func = const_cast<void *>(level_kernel(e->level_gemm[l]));
@@ -688,9 +694,6 @@ static int exec_build(Exec *e, const Dag &dag, int mode, const LowerOpts &lopts,
         e->level_items = std::move(items);
         e->level_off.assign(off.begin(), off.end());
         e->level_off.push_back(e->level_items.size());
-        e->level_args[0] = (const void *)du;
-        e->level_args[1] = (const void *)diu;
-        e->level_args[2] = (const void *)ditems;
         if (nnode)
             HIPCHK(hipGraphInstantiate(&e->gexec, e->graph, nullptr, nullptr, 0));
         *out = e;
@@ -882,11 +885,8 @@ int exec_launch_level(Exec *e, int level, hipStream_t s, std::string &err)
         err = "exec_launch_level: tiled executables only, level out of range";
         return -1;
     }
-    const UnitDesc *du = (const UnitDesc *)e->level_args[0];
-    const uint32_t *diu = (const uint32_t *)e->level_args[1];
-    const uint32_t *first = (const uint32_t *)e->level_args[2] + e->level_off[level];
     const unsigned n = (unsigned)(e->level_off[level + 1] - e->level_off[level]);
-    void *args[] = {(void *)&du, (void *)&diu, (void *)&first};
+    void *args[] = {(void *)&e->level_args[level]};
     HIPCHK(hipLaunchKernel(level_kernel(e->level_gemm[level]), dim3(n),
                            dim3((unsigned)level_threads(e->level_gemm[level])),
                            args, 0, s));

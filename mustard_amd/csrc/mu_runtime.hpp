@@ -63,7 +63,7 @@ struct Exec {
     std::vector<size_t> level_off;
     std::vector<char> level_gemm;    // LEVEL_*: the kernel the level runs on
     std::vector<double> level_flops; // algorithmic flops of the units of each level
-    const void *level_args[3] = {nullptr, nullptr, nullptr};
+    std::vector<NodeArgs> level_args;
 };
 
 int exec_create(const Dag &dag, int mode, const LowerOpts &lopts, const ExecOpts &eopts,

@@ -106,6 +106,20 @@ struct UnitDesc {
 };
 static_assert(sizeof(UnitDesc) == 128, "UnitDesc must stay 128 bytes");
 
+// The items of one graph node, passed to its kernel by value.  Workgroup b of
+// a node of one unit -- nearly every node of a factorization's serial chain --
+// runs item b of `one`, which arrives with the kernel's arguments; a node of
+// several units looks its item up (items[b], then the unit): two dependent
+// reads of memory that a cold cache serves.
+struct NodeItem {
+    uint32_t unit, item;
+};
+struct NodeArgs {
+    const UnitDesc *units;
+    const NodeItem *items;  // null: one unit
+    UnitDesc one;
+};
+
 // Per-run mutable scheduler state, all in device memory.  The words an idle
 // worker looks at come first, in one 128-byte line that one load of a wave
 // covers; the counters that claims and producers update sit in lines of
