@@ -655,17 +655,20 @@ struct Builder {
             t.c = zr ? op.c + (size_t)m0(p) * ldz : op.c + m0(p);
             if (!rec.add({p, 0}, {{p, 0}}, t))
                 return false;
-            for (int q = p + 1; q < P; q++) {
+            // the blocks after p one by one, or all of them at once
+            const int end = o.nest_panels ? std::min(p + 2, P) : P;
+            for (int q = p + 1; q < end; q++) {
+                const int mq = o.nest_panels && rev ? 0 : m0(q), nq = o.nest_panels ? n - bd[q] : sz(q);
                 OpRec g;
                 g.op = OP_GEMM;
                 g.alpha = -1.0 / op.alpha;
                 g.beta = 1.0;
                 // T_qp in memory: S(mq, mp) or, read transposed, S(mp, mq)^T
-                const double *s_qp = tt ? op.a + m0(p) + (size_t)m0(q) * lda
-                                        : op.a + m0(q) + (size_t)m0(p) * lda;
+                const double *s_qp = tt ? op.a + m0(p) + (size_t)mq * lda
+                                        : op.a + mq + (size_t)m0(p) * lda;
                 if (!zr) {
                     // Z[q rows] -= T_qp Z[p rows]
-                    g.m = sz(q);
+                    g.m = nq;
                     g.n = op.n;
                     g.k = sz(p);
                     g.a = s_qp;
@@ -673,19 +676,19 @@ struct Builder {
                     g.flags = tt ? F_TA : 0;
                     g.b = op.c + m0(p);
                     g.ldb = (int)ldz;
-                    g.c = op.c + m0(q);
+                    g.c = op.c + mq;
                     g.ldc = (int)ldz;
                 } else {
                     // B[:, q] -= B[:, p] T_qp^T
                     g.m = op.n;
-                    g.n = sz(q);
+                    g.n = nq;
                     g.k = sz(p);
                     g.a = op.c + (size_t)m0(p) * ldz;
                     g.lda = (int)ldz;
                     g.b = s_qp;
                     g.ldb = (int)lda;
                     g.flags = tt ? 0 : F_TB;
-                    g.c = op.c + (size_t)m0(q) * ldz;
+                    g.c = op.c + (size_t)mq * ldz;
                     g.ldc = (int)ldz;
                 }
                 if (!rec.add({q, 0}, {{p, 0}, {q, 0}}, g))
