@@ -247,20 +247,19 @@ def main():
         # the panel solves and diagonal factorizations beside it; hbm_gbs =
         # their HBM bytes per launch from the same counter passes as
         # `traffic` / this run's live average launch time
-        pmc_name = {"k_batch_trsm_256": "k_batch_trsm_mid"}
         others = {}
         for name, o in per.items():
             if name == "k_batch_gemm":
                 continue
             e = {"launches": o["launches"], "ms": round(o["ms"], 3),
                  "tflops": round(o["flops"] / (o["ms"] * 1e-3) * 1e-12, 3)}
-            nb = per_bytes.get(pmc_name.get(name, name))
+            nb = per_bytes.get(name)
             if nb:
                 e["hbm_bytes_per_launch"] = nb
                 e["hbm_gbs"] = round(nb * o["launches"] / (o["ms"] * 1e-3) * 1e-9, 1)
                 e["hbm_frac"] = round(e["hbm_gbs"] / PEAK_HBM_GBS, 4)
-            if pmc_name.get(name, name) in per_util:
-                e["mfma_util_pmc"] = per_util[pmc_name.get(name, name)]
+            if name in per_util:
+                e["mfma_util_pmc"] = per_util[name]
             others[name] = e
         out["roofline"]["other_kernels"] = others
         for name, p in per.items():
