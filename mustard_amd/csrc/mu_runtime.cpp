@@ -352,7 +352,11 @@ int run_units(const Lowered &low, hipStream_t s, std::string &err)
     for (const UnitDesc &d : low.units) {
         if (d.nitems <= 0)
             continue;
-        if (launch_unit(can_split(d, d.nitems) ? split_panels(d) : d, s) != 0)
+        // k_unit's LDS leaves one workgroup per CU, so the split panels of a
+        // large call run in turns of 256.  Two turns still win (order 250,
+        // 8000 right-hand sides: 31 against 38 us), four do not (16000: 59
+        // against 44 us).
+        if (launch_unit(can_split(d, 2 * d.nitems) ? split_panels(d) : d, s) != 0)
             HIPCHK(hipGetLastError());
     }
     return 0;
