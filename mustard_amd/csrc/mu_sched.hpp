@@ -152,6 +152,10 @@ MU_HD void sched_push_unit(const ExecView &ev, uint32_t u)
 // over or aborted.  Rings are tried in priority order.  One load of the wave
 // brings the four ring counts, the progress counter and the abort word, so
 // a poll is one memory round trip and an item of any priority is seen by it.
+// A worker that comes from an item claims at once: the next item of the
+// serial chain goes to the first worker that becomes free.  Workers that have
+// found nothing are many and draw lots, for the highest ring with items only:
+// a lost lot is drawn again and never turns into an item of lower priority.
 // `calls` counts the calls of this workgroup.
 template <class AT>
 MU_HD int sched_pop(const ExecView &ev, uint32_t &calls)
@@ -161,7 +165,8 @@ MU_HD int sched_pop(const ExecView &ev, uint32_t &calls)
     uint64_t t0 = 0, idle = 0;
     uint32_t seen = 0, polls = 0;
     bool first = true;
-    uint32_t tries = 0;  // polls that saw an item since the last one that saw none
+    bool waited = false;  // a poll of this call has claimed nothing
+    uint32_t tries = 0;   // lots lost since the last poll that saw no item
     for (;;) {
         const SchedPeek s = AT::peek(ev.st);
         if (s.abort)
@@ -175,8 +180,8 @@ MU_HD int sched_pop(const ExecView &ev, uint32_t &calls)
             // claim as there are items, twice as many on every further poll
             // (all of them taking and giving back the count cost 50 us and
             // more per push in the nested factorizations)
-            if (!AT::lot((uint32_t)s.cnt[p], tries))
-                continue;
+            if (waited && !AT::lot((uint32_t)s.cnt[p], tries))
+                break;
             uint32_t *cnt = reinterpret_cast<uint32_t *>(&ev.st->cnt[p]);
             if ((int32_t)w_add<AT>(cnt, 0xffffffffu) <= 0) {
                 w_add<AT>(cnt, 1u);  // none left after all: give the unit back
@@ -197,7 +202,8 @@ MU_HD int sched_pop(const ExecView &ev, uint32_t &calls)
                 AT::pause();
             }
         }
-        tries = any ? (tries < 16 ? tries + 1 : 16) : 0;
+        tries = !any || !waited ? 0 : tries < 16 ? tries + 1 : 16;
+        waited = true;
         // nothing claimed: finish, stop, or wait with the watchdog armed
         if (s.done >= ev.nitems)
             return -1;

@@ -28,6 +28,7 @@ namespace mu {
 namespace {
 
 std::atomic<int> g_producer_delay_us{0};
+std::atomic<uint32_t> g_workgroups{1};
 
 struct HostAtom {
     static bool lane0() { return true; }
@@ -42,7 +43,15 @@ struct HostAtom {
         r.abort = __atomic_load_n(&st->abort, __ATOMIC_RELAXED);
         return r;
     }
-    static bool lot(uint32_t, uint32_t) { return true; }
+    // the chance the kernel gives, 2^(tries + 1) cnt / workgroups
+    static bool lot(uint32_t cnt, uint32_t tries)
+    {
+        static std::atomic<uint32_t> seed{1};
+        thread_local uint32_t r = seed.fetch_add(1) * 0x9e3779b9u;
+        r = r * 1664525u + 1013904223u;
+        return ((uint64_t)g_workgroups.load(std::memory_order_relaxed) * (r >> 8) >> 24) <
+               ((uint64_t)cnt << (tries + 1));
+    }
     static uint32_t load_acquire(uint32_t *p) { return __atomic_load_n(p, __ATOMIC_ACQUIRE); }
     static uint32_t load_system(uint32_t *p) { return __atomic_load_n(p, __ATOMIC_ACQUIRE); }
     static void store(uint32_t *p, uint32_t v) { __atomic_store_n(p, v, __ATOMIC_RELAXED); }
@@ -266,6 +275,7 @@ bool emulate(const Dag &dag, const LowerOpts &lo, const EmuOpts &eo, EmuResult &
     chk.task_now = &task_now;
 
     g_producer_delay_us.store(eo.producer_delay_us);
+    g_workgroups.store((uint32_t)wgs);
     const int waves = 4;
     std::vector<HostWg *> wg;
     for (int g = 0; g < wgs; g++)
