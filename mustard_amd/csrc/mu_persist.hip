@@ -150,6 +150,7 @@ struct DevWave {
     const ExecView &ev;
     int *s_item;
     int *s_last;
+    __device__ __forceinline__ uint32_t id() const { return blockIdx.x; }
     __device__ __forceinline__ int wave() const
     {
         return (int)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

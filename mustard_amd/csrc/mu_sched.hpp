@@ -113,13 +113,29 @@ MU_HD void sched_abort(const ExecView &ev, uint32_t code)
 // so no worker reads it on its way to an item: a waiting worker reads it on
 // every SCHED_HOST_POLLS-th poll (about once a millisecond; with 512 workers
 // polling it every time, an order-6000 LU took 147 ms, most of it waiting
-// behind these reads), a busy one on every 256th item.
-constexpr uint32_t SCHED_HOST_POLLS = 1024;
+// behind these reads), a busy one on every 256th item.  The workers' counts
+// start SCHED_HOST_POLLS / grid apart or so, and the first to see the word
+// stores it in the state, where every poll looks: a busy run of 512 workers
+// stops after about as many items.
+constexpr uint32_t SCHED_HOST_POLLS = 1024, SCHED_HOST_ITEM = SCHED_HOST_POLLS / 256;
 
+// Worker `id`'s count at the start.
+MU_HD uint32_t sched_first_count(uint32_t id) { return (id * 389u) % SCHED_HOST_POLLS; }
+
+// Adds `step` to this workgroup's count of polls (1) and items
+// (SCHED_HOST_ITEM); when it is due, looks at the host's word and stops the
+// run if that is set.
 template <class AT>
-MU_HD bool sched_host_stopped(const ExecView &ev)
+MU_HD bool sched_host_stopped(const ExecView &ev, uint32_t &count, uint32_t step)
 {
-    return ev.host_abort && AT::bcast(AT::load_system(ev.host_abort)) != 0;
+    const uint32_t before = count;
+    count += step;
+    if ((before ^ count) < SCHED_HOST_POLLS)
+        return false;
+    if (!ev.host_abort || AT::bcast(AT::load_system(ev.host_abort)) == 0)
+        return false;
+    sched_abort<AT>(ev, 4u);
+    return true;
 }
 
 // The run was aborted, by the device watchdog or by the host (the latter
@@ -129,7 +145,7 @@ MU_HD bool sched_stopped(const ExecView &ev, uint32_t &polls)
 {
     if (w_load<AT>(&ev.st->abort))
         return true;
-    return (++polls & (SCHED_HOST_POLLS - 1)) == 0 && sched_host_stopped<AT>(ev);
+    return sched_host_stopped<AT>(ev, polls, 1);
 }
 
 // Queue all items of unit u on its priority ring (one thread).
@@ -156,14 +172,14 @@ MU_HD void sched_push_unit(const ExecView &ev, uint32_t u)
 // serial chain goes to the first worker that becomes free.  Workers that have
 // found nothing are many and draw lots, for the highest ring with items only:
 // a lost lot is drawn again and never turns into an item of lower priority.
-// `calls` counts the calls of this workgroup.
+// `count` is this workgroup's count of sched_host_stopped.
 template <class AT>
-MU_HD int sched_pop(const ExecView &ev, uint32_t &calls)
+MU_HD int sched_pop(const ExecView &ev, uint32_t &count)
 {
-    if ((++calls & 255u) == 0 && sched_host_stopped<AT>(ev))
+    if (sched_host_stopped<AT>(ev, count, SCHED_HOST_ITEM))
         return -1;
     uint64_t t0 = 0, idle = 0;
-    uint32_t seen = 0, polls = 0;
+    uint32_t seen = 0;
     bool first = true;
     bool waited = false;  // a poll of this call has claimed nothing
     uint32_t tries = 0;   // lots lost since the last poll that saw no item
@@ -197,7 +213,7 @@ MU_HD int sched_pop(const ExecView &ev, uint32_t &calls)
                 const uint32_t v = w_load_acquire<AT>(ev.slots[p] + pos);
                 if (v)
                     return (int)(v - 1);
-                if (sched_stopped<AT>(ev, polls))
+                if (sched_stopped<AT>(ev, count))
                     return -1;
                 AT::pause();
             }
@@ -207,7 +223,7 @@ MU_HD int sched_pop(const ExecView &ev, uint32_t &calls)
         // nothing claimed: finish, stop, or wait with the watchdog armed
         if (s.done >= ev.nitems)
             return -1;
-        if ((++polls & (SCHED_HOST_POLLS - 1)) == 0 && sched_host_stopped<AT>(ev))
+        if (sched_host_stopped<AT>(ev, count, 1))
             return -1;
         const uint64_t now = AT::now();
         if (first || s.done != seen) {
@@ -234,14 +250,13 @@ MU_HD int sched_pop(const ExecView &ev, uint32_t &calls)
 // The wait ends when executing items finish, so it always ends; false when
 // the run was aborted.
 template <class AT>
-MU_HD bool sched_admit(const ExecView &ev, int task)
+MU_HD bool sched_admit(const ExecView &ev, int task, uint32_t &count)
 {
     if (ev.task_cap <= 0 || task < 0)
         return true;
     uint32_t *run = reinterpret_cast<uint32_t *>(ev.task_running + task);
     uint32_t *occ = reinterpret_cast<uint32_t *>(&ev.st->occ);
     const uint32_t share = (uint32_t)ev.task_budget;
-    uint32_t polls = 0;
     for (;;) {
         const uint32_t r = w_load<AT>(run);
         if (r > 0 && r < (uint32_t)ev.task_cap) {
@@ -257,7 +272,7 @@ MU_HD bool sched_admit(const ExecView &ev, int task)
                 w_add<AT>(occ, (uint32_t)(-(int32_t)share));
             }
         }
-        if (sched_stopped<AT>(ev, polls))
+        if (sched_stopped<AT>(ev, count))
             return false;
         AT::pause();
     }
@@ -298,16 +313,17 @@ MU_HD void sched_release(const ExecView &ev, uint32_t u, uint32_t first, uint32_
 // The worker loop of one workgroup (replaces kernel_scheduler,
 // mustard/mustard.h:108-129; there one thread device-launches a sub-graph
 // per task, here every workgroup runs items inline).  W is the per-wave
-// context: wave() (uniform), barrier(), the two LDS words set_item/item and
-// set_last/last, fence_release(), threads(f) calling f(first, stride) for
-// each thread the caller stands for, and the item body run(d, item).
+// context: id() (the workgroup), wave() (uniform), barrier(), the two LDS
+// words set_item/item and set_last/last, fence_release(), threads(f) calling
+// f(first, stride) for each thread the caller stands for, and the item body
+// run(d, item).
 template <class AT, class W>
 MU_HD void sched_worker(const ExecView &ev, W &w)
 {
-    uint32_t calls = 0;  // sched_pop calls of this workgroup (wave 0)
+    uint32_t count = sched_first_count(w.id());  // of sched_host_stopped (wave 0)
     if (w.wave() == 0) {
-        int it = sched_pop<AT>(ev, calls);
-        if (it >= 0 && !sched_admit<AT>(ev, ev.units[ev.item_unit[it]].task))
+        int it = sched_pop<AT>(ev, count);
+        if (it >= 0 && !sched_admit<AT>(ev, ev.units[ev.item_unit[it]].task, count))
             it = -1;
         w.set_item(it);
     }
@@ -336,8 +352,8 @@ MU_HD void sched_worker(const ExecView &ev, W &w)
             sched_retire<AT>(ev, ev.units[u].task);
             if (last)
                 w_add_release<AT>(&ev.st->done, (uint32_t)ev.units[u].nitems);
-            int it = sched_pop<AT>(ev, calls);
-            if (it >= 0 && !sched_admit<AT>(ev, ev.units[ev.item_unit[it]].task))
+            int it = sched_pop<AT>(ev, count);
+            if (it >= 0 && !sched_admit<AT>(ev, ev.units[ev.item_unit[it]].task, count))
                 it = -1;
             w.set_item(it);
         }

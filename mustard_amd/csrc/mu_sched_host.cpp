@@ -115,7 +115,8 @@ class WgBarrier {
 };
 
 struct HostWg {
-    explicit HostWg(int waves) : bar(waves) {}
+    HostWg(int id, int waves) : id((uint32_t)id), bar(waves) {}
+    uint32_t id;
     WgBarrier bar;
     int s_item = -1, s_last = 0;  // the workgroup's two LDS words
 };
@@ -141,6 +142,8 @@ struct Check {
     // would count the task twice
     std::mutex task_mu;
     int body_barriers = 2;
+    std::atomic<uint64_t> started{0};
+    uint64_t abort_after = 0;
 };
 
 struct HostWave {
@@ -148,6 +151,7 @@ struct HostWave {
     HostWg &wg;
     Check &chk;
     int w;
+    uint32_t id() const { return wg.id; }
     int wave() const { return w; }
     void barrier() { wg.bar.wait(); }
     void set_item(int v) { wg.s_item = v; }
@@ -169,6 +173,8 @@ struct HostWave {
                 if (__atomic_load_n(&chk.left[p], __ATOMIC_ACQUIRE) != 0)
                     chk.violations++;
             (*chk.runs)[item]++;
+            if (++chk.started == chk.abort_after)
+                __atomic_store_n(ev.host_abort, 1u, __ATOMIC_RELEASE);
             if (task >= 0 && task < (int)chk.task_now->size()) {
                 std::lock_guard<std::mutex> g(chk.task_mu);
                 const int32_t now = ++(*chk.task_now)[task];
@@ -273,13 +279,14 @@ bool emulate(const Dag &dag, const LowerOpts &lo, const EmuOpts &eo, EmuResult &
     chk.left = left.data();
     chk.runs = &runs;
     chk.task_now = &task_now;
+    chk.abort_after = eo.abort_after_items;
 
     g_producer_delay_us.store(eo.producer_delay_us);
     g_workgroups.store((uint32_t)wgs);
     const int waves = 4;
     std::vector<HostWg *> wg;
     for (int g = 0; g < wgs; g++)
-        wg.push_back(new HostWg(waves));
+        wg.push_back(new HostWg(g, waves));
     std::vector<std::thread> pool;
     for (int g = 0; g < wgs; g++)
         for (int w = 0; w < waves; w++)

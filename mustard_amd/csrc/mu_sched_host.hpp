@@ -12,6 +12,7 @@ struct EmuOpts {
     int workgroups = 8;          // emulated workgroups (four threads each)
     double timeout_s = 20.0;     // device watchdog: no progress for this long
     double host_deadline_s = 0;  // host watchdog: abort after this long (0 = none)
+    uint64_t abort_after_items = 0;  // host abort once this many items have started (0 = none)
     int bump_unit = -1;          // >= 0: one never-satisfied dependency on this unit
     int producer_delay_us = 0;   // stall of every producer between reserving and storing
     int sm = 0;                  // CU budget per task, percent (0 = none)
