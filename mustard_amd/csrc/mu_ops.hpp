@@ -1300,15 +1300,17 @@ __device__ __forceinline__ void getrf16(double (&x)[16], double (&z)[16], double
 __device__ __forceinline__ void lds_wait() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // Block (i, j) of an n x n tile into its register format; rows and columns
-// past n read the last one.  The scheduling barrier keeps one block's
-// addresses from living beside the next one's.
+// past n read the last one.  Offsets are 64-bit everywhere: a tile of a tall
+// matrix spans more than 2^32 elements from a leading dimension of 34 million
+// on.  The scheduling barrier keeps one block's addresses from living beside
+// the next one's.
 __device__ __forceinline__ void load_blk16(v4d &v, const MU_G double *a, unsigned lda, int n, int i,
                                            int j, int li, int lk)
 {
-    const unsigned r = min(16 * i + li, n - 1);
+    const size_t r = min(16 * i + li, n - 1);
 #pragma unroll
     for (int e = 0; e < 4; e++)
-        v[e] = a[r + (unsigned)min(16 * j + 4 * e + lk, n - 1) * lda];
+        v[e] = a[r + (size_t)min(16 * j + 4 * e + lk, n - 1) * lda];
     __builtin_amdgcn_sched_barrier(0);
 }
 
@@ -1357,7 +1359,7 @@ __device__ __forceinline__ void store_blk16(const SmallCtx &c, int i, const v4d 
     if (16 * i + c.li < c.n)
 #pragma unroll
         for (int e = 0; e < 4; e++)
-            (c.a + 16 * i + (size_t)(16 * P + 4 * e) * c.lda)[c.li + c.lk * c.lda] = x[e];
+            (c.a + 16 * i + (size_t)(16 * P + 4 * e) * c.lda)[c.li + (size_t)c.lk * c.lda] = x[e];
 }
 
 // The owner of block row p + 1 hands its diagonal block to the factoring wave.
@@ -1387,7 +1389,7 @@ __device__ __forceinline__ void store_diag16(const SmallCtx &c, int p, const dou
         for (int e = 0; e < 4; e++) {
             const int k = 4 * e + c.lk;
             if (LOWER ? k <= c.li : 16 * p + k < c.n)
-                (c.a + 16 * p + (size_t)(16 * p + 4 * e) * c.lda)[c.li + c.lk * c.lda] =
+                (c.a + 16 * p + (size_t)(16 * p + 4 * e) * c.lda)[c.li + (size_t)c.lk * c.lda] =
                     D[c.li * BF_LD + k];
         }
 }
@@ -1616,7 +1618,7 @@ __device__ __forceinline__ void getrf_step(const SmallCtx &c, v4d (&R0)[8], v4d 
         for (int e = 0; e < 4; e++) {
             Ub[(j - 1) * 256 + e * 64 + c.lane] = -x[e];
             if (16 * j + c.li < c.n)
-                (c.a + 16 * P + 4 * e + (size_t)(16 * j) * c.lda)[c.lk + c.li * c.lda] = x[e];
+                (c.a + 16 * P + 4 * e + (size_t)(16 * j) * c.lda)[c.lk + (size_t)c.li * c.lda] = x[e];
         }
     }
     lds_barrier();  // B
