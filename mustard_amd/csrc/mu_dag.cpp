@@ -436,7 +436,7 @@ struct Builder {
                 d.gn = cdiv(op.n, 4 * TRSM_W);
                 // one item either way, and the four waves share it (launches of
                 // few wider panels are split where they are put together)
-                if (op.m <= TRSM_REG_MAX && op.n <= TRSM_W)
+                if (op.m <= TRSM_REG_MAX && op.n <= TRSM_W && op.lda < TRSM_SPLIT_LD)
                     d.flags |= F_SPLIT;
                 if (op.m > TRSM_REG_MAX) {
                     d.gn = cdiv(op.n, TRSM_W);

@@ -1965,7 +1965,7 @@ __device__ __attribute__((always_inline)) inline void trsm_panel_reg(const UnitD
     const int nlast = n - 16 * (nb - 1);
     MU_G double *zb = z + (size_t)pc * zcs;
     // row 16 i + 4 e + lk, column lic: a uniform part and this lane's
-    const unsigned zl = (rev ? 3 - lk : lk) * zrs + lic * zcs;
+    const size_t zl = (size_t)(rev ? 3 - lk : lk) * zrs + (size_t)lic * zcs;
     auto zrow = [&](int r) -> size_t {  // of rows r .. r + 3, the lowest address
         return (size_t)(rev ? n - 4 - r : r) * zrs;
     };

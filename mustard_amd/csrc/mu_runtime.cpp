@@ -277,7 +277,8 @@ constexpr int TRSM_SPLIT_ITEMS = 256;
 
 static bool can_split(const UnitDesc &d, int launch_items)
 {
-    return d.op == OP_TRSM && !(d.flags & (F_INV | F_SPLIT)) && launch_items < TRSM_SPLIT_ITEMS;
+    return d.op == OP_TRSM && !(d.flags & (F_INV | F_SPLIT)) && launch_items < TRSM_SPLIT_ITEMS &&
+           d.lda < TRSM_SPLIT_LD;
 }
 static UnitDesc split_panels(UnitDesc d)
 {

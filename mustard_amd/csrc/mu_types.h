@@ -55,8 +55,8 @@ enum Flag : int32_t {
     F_CVT_BOTH = 1 << 16, // CVT with F_CVT_T: also stores the block untransposed at (a, lda)
     F_BROW = 1 << 17,    // F_A32 GEMM: B and C stored by rows (B(k, j) at b[k*ldb + j], C(i, j)
                          // at c[i*ldc + j])
-    F_SPLIT = 1 << 18,   // TRSM without F_INV: items are panels of <= 16 right-hand sides, each on
-                         // all four waves
+    F_SPLIT = 1 << 18,   // TRSM without F_INV, lda < TRSM_SPLIT_LD: items are panels of <= 16
+                         // right-hand sides, each on all four waves
 };
 
 // Kernel geometry (fixed for gfx950: 4 waves of 64 lanes per workgroup).
@@ -67,6 +67,8 @@ constexpr int GEMM_BK = 8;      // k-block staged in LDS per step
 constexpr int TRSM_W = 16;        // right-hand sides per wave (F_INV: per workgroup) of a TRSM item
 constexpr int TRSM_REG_MAX = 256; // largest triangle a TRSM item solves in registers, 4 * TRSM_W
                                   // right-hand sides per item; larger ones (F_INV) in LDS
+constexpr int TRSM_SPLIT_LD = 1 << 25; // F_SPLIT: leading dimension of the triangle below this (a
+                                  // lane's byte offset in a 16 x 16 block is 32-bit)
 constexpr int TRSM_NMAX = 1024;   // largest triangle a TRSM item keeps in LDS
 constexpr int TRSM_NEST = 256;    // default: triangles above this order nest into blocks,
                                   // whose solves run beside GEMM workgroups on a CU
