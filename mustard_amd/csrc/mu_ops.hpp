@@ -1068,9 +1068,10 @@ __device__ __forceinline__ void report_info(const UnitDesc &u, int col)
 //     a row_newbcast operand) instead of two readlanes per element;
 //   * the same wave forms the inverse(s) of the factored block with the same
 //     instruction, so every other block of the panel is one product with a
-//     16 x 16 inverse on MFMA instead of a sweep over its rows;
+//     16 x 16 inverse on MFMA, corrected once (solve_blk16), instead of a
+//     sweep over its rows;
 //   * the trailing update is MFMA on registers.
-// Alone, order 125: POTRF 37 -> 24 us, GETRF 91 -> 38 us against the form that
+// Alone, order 125: POTRF 37 -> 27 us, GETRF 91 -> 38 us against the form that
 // swept all 128 rows with readlanes and kept inv(L11) only.
 //
 // Registers: block (i, j) lives on the wave of its block row (rows w and
@@ -1337,6 +1338,42 @@ __device__ __forceinline__ void update_row(v4d *acc, const double *lds, const v4
     }
 }
 
+// X = inv(T) Y for N blocks of Y in register format, T a lower 16 x 16
+// triangle: W ~ inv(T) and T come as this lane's MFMA A operands, element
+// (li, 4 e + lk).  The product with an inverse alone leaves a residual of eps
+// cond(T) where substitution leaves eps -- a Cholesky of a kernel matrix (128
+// points, 1e-12 added to the diagonal) then met a negative pivot -- so it is
+// corrected once, X += W (Y - T X): the residual falls to eps + (eps
+// cond(T))^2.  Eight more MFMAs per block (POTRF of order 128: 29.0 -> 32.2 us
+// in a graph node); substituting takes 136 instructions on the vector ALU, each
+// of which waits behind the MFMAs of the GEMM workgroups on its SIMD.
+template <int N>
+__device__ __forceinline__ void solve_blk16(v4d (&X)[N], const v4d (&Y)[N], const double (&w)[4],
+                                            const double (&t)[4])
+{
+    v4d R[N];
+#pragma unroll
+    for (int b = 0; b < N; b++) {
+        X[b] = v4d{0.0, 0.0, 0.0, 0.0};
+        R[b] = Y[b];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int b = 0; b < N; b++)
+            X[b] = mfma_f64(w[e], Y[b][e], X[b]);
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int b = 0; b < N; b++)
+            R[b] = mfma_f64(t[e], -X[b][e], R[b]);
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int b = 0; b < N; b++)
+            X[b] = mfma_f64(w[e], R[b][e], X[b]);
+}
+
 struct SmallCtx {
     int n, nb, w, li, lk, lane;
     MU_G double *a;
@@ -1416,23 +1453,38 @@ __device__ __forceinline__ void potrf_diag(const SmallCtx &c, const UnitDesc &u,
         D[li * BF_LD + k] = x[k];
 }
 
-// Tile waves, step P: L_ip^T = inv(L_pp) A_ip^T for the blocks below, stored
-// and handed on as -L_ip (Lb); then A_ij^T += (-L_jp) L_ip^T, the next
+// Tile waves, step P: L_ip^T = inv(L_pp) A_ip^T for the blocks below (D: L_pp
+// with anything above its diagonal), stored and handed on as -L_ip (Lb); then A_ij^T += (-L_jp) L_ip^T, the next
 // diagonal block first.  R0: row w, columns 0 .. 3; R1: row w + 4 (blocks
 // right of the diagonal hold nothing that is read).
 template <int P, bool W0>
 __device__ __forceinline__ void potrf_step(const SmallCtx &c, v4d (&R0)[4], v4d (&R1)[8],
-                                           double *W, double *Lb)
+                                           double *W, const double *D, double *Lb)
 {
     const bool on0 = !W0 && P < 3 && c.w > P && c.w < c.nb;
     const bool on1 = c.w + 4 > P && c.w + 4 < c.nb;
-    v4d X0 = {0.0, 0.0, 0.0, 0.0}, X1 = X0;
+    v4d X0, X1;
+    double wv[4], tv[4];
 #pragma unroll
-    for (int e = 0; e < 4; e++) {  // a finished row solves a block nothing reads
-        const double wv = W[c.li * BF_LD + 4 * e + c.lk];
-        if constexpr (!W0 && P < 3)
-            X0 = mfma_f64(wv, R0[P][e], X0);
-        X1 = mfma_f64(wv, R1[P][e], X1);
+    for (int e = 0; e < 4; e++) {
+        const int k = 4 * e + c.lk;
+        wv[e] = W[c.li * BF_LD + k];
+        tv[e] = k <= c.li ? D[c.li * BF_LD + k] : 0.0;
+    }
+    if constexpr (!W0 && P < 3) {
+        if (on0) {  // row w + 4 may be past the tile: a block nothing reads
+            v4d X[2];
+            const v4d Y[2] = {R0[P], R1[P]};
+            solve_blk16(X, Y, wv, tv);
+            X0 = X[0];
+            X1 = X[1];
+        }
+    }
+    if (!on0 && on1) {
+        v4d X[1];
+        const v4d Y[1] = {R1[P]};
+        solve_blk16(X, Y, wv, tv);
+        X1 = X[0];
     }
     auto put = [&](int i, const v4d &x) {
 #pragma unroll
@@ -1480,16 +1532,16 @@ __device__ __forceinline__ void potrf_step(const SmallCtx &c, v4d (&R0)[4], v4d 
 // Step p (a switch: the register arrays need constant indices).
 template <bool W0>
 __device__ __forceinline__ void potrf_steps(const SmallCtx &c, int p, v4d (&R0)[4], v4d (&R1)[8],
-                                            double *W, double *Lb)
+                                            double *W, const double *D, double *Lb)
 {
     switch (p) {
-    case 0: potrf_step<0, W0>(c, R0, R1, W, Lb); break;
-    case 1: potrf_step<1, W0>(c, R0, R1, W, Lb); break;
-    case 2: potrf_step<2, W0>(c, R0, R1, W, Lb); break;
-    case 3: potrf_step<3, W0>(c, R0, R1, W, Lb); break;
-    case 4: potrf_step<4, W0>(c, R0, R1, W, Lb); break;
-    case 5: potrf_step<5, W0>(c, R0, R1, W, Lb); break;
-    default: potrf_step<6, W0>(c, R0, R1, W, Lb); break;
+    case 0: potrf_step<0, W0>(c, R0, R1, W, D, Lb); break;
+    case 1: potrf_step<1, W0>(c, R0, R1, W, D, Lb); break;
+    case 2: potrf_step<2, W0>(c, R0, R1, W, D, Lb); break;
+    case 3: potrf_step<3, W0>(c, R0, R1, W, D, Lb); break;
+    case 4: potrf_step<4, W0>(c, R0, R1, W, D, Lb); break;
+    case 5: potrf_step<5, W0>(c, R0, R1, W, D, Lb); break;
+    default: potrf_step<6, W0>(c, R0, R1, W, D, Lb); break;
     }
 }
 
@@ -1530,7 +1582,7 @@ __device__ __forceinline__ void potrf_waves(SmallCtx c, const UnitDesc &u, doubl
             potrf_diag(c, u, p, W, D + (p & 1) * BF_BLK);
         lds_barrier();  // A
         if (p + 1 < nb)
-            potrf_steps<W0>(c, p, R0, R1, W, Lb);
+            potrf_steps<W0>(c, p, R0, R1, W, D + (p & 1) * BF_BLK, Lb);
         if (w == (p & 3))
             store_diag16<true>(c, p, D + (p & 1) * BF_BLK);
         if (p + 1 == nb)
