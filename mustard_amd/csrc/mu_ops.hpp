@@ -1071,7 +1071,7 @@ __device__ __forceinline__ void report_info(const UnitDesc &u, int col)
 //     16 x 16 inverse on MFMA, corrected once (solve_blk16), instead of a
 //     sweep over its rows;
 //   * the trailing update is MFMA on registers.
-// Alone, order 125: POTRF 37 -> 27 us, GETRF 91 -> 38 us against the form that
+// Alone, order 125: POTRF 37 -> 27 us, GETRF 91 -> 47 us against the form that
 // swept all 128 rows with readlanes and kept inv(L11) only.
 //
 // Registers: block (i, j) lives on the wave of its block row (rows w and
@@ -1272,28 +1272,40 @@ __device__ __forceinline__ void potrf16(double (&x)[16], double (&z)[16], double
     }
 }
 
-// No-pivot elimination of a 16 x 16 block, lane li holding row li in x:
-// afterwards x[c] is the multiplier for c < li (unit lower factor) and the
-// upper factor's row otherwise; z as above for the unit lower factor, row C
-// stored to W scaled by 1 / pivot in the lanes with `scale`.
+// No-pivot elimination of a 16 x 16 block, A = L U, and inv(L) or inv(U)^T.
+// Lane li of a group of 16 holds row li of the block in x (ROW) or column li
+// (!ROW), afterwards the same of the packed factors.  Both forms round alike,
+// l = fl(a / pivot) and a - l u in one FMA, so they hold the same factors to
+// the bit: scaling the transposed block's rows by the pivot instead (an
+// elimination of A^T) gives another U, and its inverse is off by eps cond(A).
+// Column C: the multipliers l (ROW), or the pivot row u, are in m; lane C has
+// the other one, in place (ROW) or scaled by 1 / pivot first (!ROW).
+// z: column li of the identity, turned into the inverse's by substitution
+// with L, or U^T (!ROW), row C of it stored to W.
 template <int C>
 __device__ __forceinline__ void getrf16(double (&x)[16], double (&z)[16], double *W, double piv,
-                                        int li, bool scale, int &bad)
+                                        int li, bool row, int &bad)
 {
     if constexpr (C < 16) {
         bad = min(bad, piv == 0.0 ? C : 16);
         const double rd = rcp_nr(piv);
-        const double m = li > C ? x[C] * rd : 0.0;
+        const double rr = row ? rd : 1.0, rc = row ? 1.0 : rd;
+        const double m = li > C ? x[C] * rr : 0.0;
         x[C] = li > C ? m : x[C];
+        const double f = li == C ? rc : 1.0;
+#pragma unroll
+        for (int k = C + 1; k < 16; k++)
+            x[k] *= f;
         if constexpr (C < 15) {
             col_head<true, C>(x, m, m);
             piv = bcast16<C + 1>(x[C + 1]);
         }
-        W[C * BF_LD] = scale ? z[C] * rd : z[C];
+        z[C] *= rc;
+        W[C * BF_LD] = z[C];
         if constexpr (C < 13)
             fms_self<C, C + 4>(x, m);
         fms_lane<C + 1>(z, m, z[C]);
-        getrf16<C + 1>(x, z, W, piv, li, scale, bad);
+        getrf16<C + 1>(x, z, W, piv, li, row, bad);
     }
 }
 
@@ -1344,9 +1356,10 @@ __device__ __forceinline__ void update_row(v4d *acc, const double *lds, const v4
 // cond(T) where substitution leaves eps -- a Cholesky of a kernel matrix (128
 // points, 1e-12 added to the diagonal) then met a negative pivot -- so it is
 // corrected once, X += W (Y - T X): the residual falls to eps + (eps
-// cond(T))^2.  Eight more MFMAs per block (POTRF of order 128: 29.0 -> 32.2 us
-// in a graph node); substituting takes 136 instructions on the vector ALU, each
-// of which waits behind the MFMAs of the GEMM workgroups on its SIMD.
+// cond(T))^2.  That is eight more MFMAs per block; substitution is 136
+// instructions on the vector ALU, each of which waits behind the MFMAs of the
+// GEMM workgroups on its SIMD.  Order 128 in a graph node: POTRF 29.0 -> 32.2
+// us, GETRF 39.0 -> 46.9 us (1.9 of these for getrf16's consistent factors).
 template <int N>
 __device__ __forceinline__ void solve_blk16(v4d (&X)[N], const v4d (&Y)[N], const double (&w)[4],
                                             const double (&t)[4])
@@ -1606,9 +1619,8 @@ __device__ __attribute__((always_inline)) inline void potrf_small(const UnitDesc
 }
 
 // No-pivot LU.  Factoring step p: two groups of 16 lanes eliminate A_pp at
-// once, one on the block and one on its transpose, whose unit lower factor is
-// the transposed unit upper factor of A_pp = L D U', and invert both:
-// W1 = inv(L), W2 = inv(U)^T = D^-1 inv(U')^T.  The packed factors go to D.
+// once, one on its rows and one on its columns, and invert one factor each:
+// W1 = inv(L), W2 = inv(U)^T.  The packed factors go to D.
 __device__ __forceinline__ void getrf_diag(const SmallCtx &c, const UnitDesc &u, int p, double *W1,
                                            double *W2, double *D)
 {
@@ -1623,7 +1635,7 @@ __device__ __forceinline__ void getrf_diag(const SmallCtx &c, const UnitDesc &u,
     }
     lds_wait();
     int bad = 16;
-    getrf16<0>(x, z, (g ? W2 : W1) + li, bcast16<0>(x[0]), li, g != 0, bad);
+    getrf16<0>(x, z, (g ? W2 : W1) + li, bcast16<0>(x[0]), li, g == 0, bad);
     if (bad < 16 && c.lane == 0)
         report_info(u, 16 * p + bad);
     if (g == 0)
@@ -1642,35 +1654,61 @@ __device__ __forceinline__ void put_raw16(const SmallCtx &c, const v4d (&R)[8], 
             put_diag16(c, raw + (j - 1) * BF_BLK, R[j]);
 }
 
-// Tile waves, step P: L_ip^T = inv(U)^T A_ip^T for the blocks below, a share
-// of the row panel, U_pj = inv(L) A_pj (copied to LDS raw by its owner),
+// Tile waves, step P (D: the packed factors of A_pp): L_ip^T = inv(U)^T A_ip^T
+// for the blocks below, a share of the row panel, U_pj = inv(L) A_pj (copied to LDS raw by its owner),
 // handed on as -U_pj (Ub); then A_ij^T += (-U_pj)^T L_ip^T, the next diagonal
 // block first.  R0, R1: block rows w and w + 4.
 template <int P, bool W0>
 __device__ __forceinline__ void getrf_step(const SmallCtx &c, v4d (&R0)[8], v4d (&R1)[8],
-                                           double *W1, const double *W2, double *raw, double *Ub)
+                                           double *W1, const double *W2, const double *D,
+                                           double *raw, double *Ub)
 {
     const bool on0 = !W0 && P < 3 && c.w > P && c.w < c.nb;
     const bool on1 = c.w + 4 > P && c.w + 4 < c.nb;
-    v4d X0 = {0.0, 0.0, 0.0, 0.0}, X1 = X0;
+    v4d X0, X1;
+    double wv[4], tv[4];
 #pragma unroll
-    for (int e = 0; e < 4; e++) {  // a finished row solves a block nothing reads
-        const double wv = W2[c.li * BF_LD + 4 * e + c.lk];
-        if constexpr (!W0 && P < 3)
-            X0 = mfma_f64(wv, R0[P][e], X0);
-        X1 = mfma_f64(wv, R1[P][e], X1);
+    for (int e = 0; e < 4; e++) {
+        const int k = 4 * e + c.lk;
+        wv[e] = W2[c.li * BF_LD + k];
+        tv[e] = k <= c.li ? D[k * BF_LD + c.li] : 0.0;  // U^T
     }
-    for (int j = P + 1 + c.w; j < c.nb; j += 4) {
-        const double *b = raw + (j - 1) * BF_BLK;
-        v4d x = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-            x = mfma_f64(W1[c.li * BF_LD + 4 * e + c.lk], b[(4 * e + c.lk) * BF_LD + c.li], x);
+    if constexpr (!W0 && P < 3) {
+        if (on0) {  // row w + 4 may be past the tile: a block nothing reads
+            v4d X[2];
+            const v4d Y[2] = {R0[P], R1[P]};
+            solve_blk16(X, Y, wv, tv);
+            X0 = X[0];
+            X1 = X[1];
+        }
+    }
+    if (!on0 && on1) {
+        v4d X[1];
+        const v4d Y[1] = {R1[P]};
+        solve_blk16(X, Y, wv, tv);
+        X1 = X[0];
+    }
+    if (P + 1 + c.w < c.nb) {
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            Ub[(j - 1) * 256 + e * 64 + c.lane] = -x[e];
-            if (16 * j + c.li < c.n)
-                (c.a + 16 * P + 4 * e + (size_t)(16 * j) * c.lda)[c.lk + (size_t)c.li * c.lda] = x[e];
+            const int k = 4 * e + c.lk;
+            wv[e] = W1[c.li * BF_LD + k];
+            tv[e] = k < c.li ? D[c.li * BF_LD + k] : k == c.li ? 1.0 : 0.0;  // L
+        }
+        for (int j = P + 1 + c.w; j < c.nb; j += 4) {
+            const double *b = raw + (j - 1) * BF_BLK;
+            v4d X[1], Y[1];
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                Y[0][e] = b[(4 * e + c.lk) * BF_LD + c.li];
+            solve_blk16(X, Y, wv, tv);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                Ub[(j - 1) * 256 + e * 64 + c.lane] = -X[0][e];
+                if (16 * j + c.li < c.n)
+                    (c.a + 16 * P + 4 * e + (size_t)(16 * j) * c.lda)[c.lk + (size_t)c.li * c.lda] =
+                        X[0][e];
+            }
         }
     }
     lds_barrier();  // B
@@ -1716,16 +1754,17 @@ __device__ __forceinline__ void getrf_step(const SmallCtx &c, v4d (&R0)[8], v4d 
 
 template <bool W0>
 __device__ __forceinline__ void getrf_steps(const SmallCtx &c, int p, v4d (&R0)[8], v4d (&R1)[8],
-                                            double *W1, const double *W2, double *raw, double *Ub)
+                                            double *W1, const double *W2, const double *D,
+                                            double *raw, double *Ub)
 {
     switch (p) {
-    case 0: getrf_step<0, W0>(c, R0, R1, W1, W2, raw, Ub); break;
-    case 1: getrf_step<1, W0>(c, R0, R1, W1, W2, raw, Ub); break;
-    case 2: getrf_step<2, W0>(c, R0, R1, W1, W2, raw, Ub); break;
-    case 3: getrf_step<3, W0>(c, R0, R1, W1, W2, raw, Ub); break;
-    case 4: getrf_step<4, W0>(c, R0, R1, W1, W2, raw, Ub); break;
-    case 5: getrf_step<5, W0>(c, R0, R1, W1, W2, raw, Ub); break;
-    default: getrf_step<6, W0>(c, R0, R1, W1, W2, raw, Ub); break;
+    case 0: getrf_step<0, W0>(c, R0, R1, W1, W2, D, raw, Ub); break;
+    case 1: getrf_step<1, W0>(c, R0, R1, W1, W2, D, raw, Ub); break;
+    case 2: getrf_step<2, W0>(c, R0, R1, W1, W2, D, raw, Ub); break;
+    case 3: getrf_step<3, W0>(c, R0, R1, W1, W2, D, raw, Ub); break;
+    case 4: getrf_step<4, W0>(c, R0, R1, W1, W2, D, raw, Ub); break;
+    case 5: getrf_step<5, W0>(c, R0, R1, W1, W2, D, raw, Ub); break;
+    default: getrf_step<6, W0>(c, R0, R1, W1, W2, D, raw, Ub); break;
     }
 }
 
@@ -1768,7 +1807,7 @@ __device__ __forceinline__ void getrf_waves(SmallCtx c, const UnitDesc &u, doubl
             getrf_diag(c, u, p, W1, W2, D + (p & 1) * BF_BLK);
         lds_barrier();  // A
         if (p + 1 < nb)
-            getrf_steps<W0>(c, p, R0, R1, W1, W2, raw, Ub);
+            getrf_steps<W0>(c, p, R0, R1, W1, W2, D + (p & 1) * BF_BLK, raw, Ub);
         if (w == (p & 3))
             store_diag16<false>(c, p, D + (p & 1) * BF_BLK);
         if (p + 1 == nb)

@@ -58,3 +58,15 @@ def test_cholesky_tile(torch_gpu, n, nugget, mode):
         np.linalg.cholesky(A)
         L = np.tril(factor("chol", A, mode))
         assert np.all(np.abs(product(L, L.T) - A) <= bound(n, np.abs(L) @ np.abs(L).T))
+
+
+@pytest.mark.parametrize("mode", ["eager", "tiled", "subgraph"])
+@pytest.mark.parametrize("nugget", [1e-6, 1e-8, 1e-10, 1e-12, 1e-13, None])
+@pytest.mark.parametrize("n", [17, 33, 64, 100, 125, 128])
+def test_lu_tile(torch_gpu, n, nugget, mode):
+    """Kernel matrices, and (None) uniform ones without any dominance, whose pivots and multipliers vary wildly."""
+    for seed in range(5):
+        A = np.random.default_rng(seed).uniform(-1, 1, (n, n)) if nugget is None else kernel_matrix(n, nugget, seed)
+        F = factor("lu", A, mode)
+        L, R = np.tril(F, -1) + np.eye(n), np.triu(F)
+        assert np.all(np.abs(product(L, R) - A) <= bound(n, np.abs(L) @ np.abs(R)))
