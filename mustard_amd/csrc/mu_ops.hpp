@@ -1854,7 +1854,7 @@ __device__ __attribute__((always_inline)) inline void getrf_small(const UnitDesc
 // diagonal blocks at once, one block per group of 16 lanes, so no inversion
 // kernel runs before it.  One node of the Cholesky at n = 7007, against a
 // panel of 16 right-hand sides per workgroup in LDS (a barrier per 16 rows,
-// four waves sharing each panel): order 125 28 -> 14 us, order 250 35 us
+// four waves sharing each panel): order 125 28 -> 17 us, order 250 35 us
 // after an inversion kernel of 10 us -> 38 us; N = 24000 LU 166 -> 152 ms.
 //
 // Strides are run-time values, so one body serves every side, triangle and
@@ -1876,18 +1876,94 @@ __device__ __forceinline__ T *uniform_ptr(T *p)
     return (T *)(((unsigned long long)hi << 32) | lo);
 }
 
+// Triangles of order <= SMALL_MAX are solved with the correction of
+// solve_blk16, to the backward error of substitution; larger ones (parts of
+// whole tiles) with the inverses of their diagonal blocks alone.  The
+// correction costs (order 125, eager calls) 8.1 -> 10.2 us on panels of 16
+// right-hand sides and 17.4 -> 20.4 us for 16384 on panels of 64.  The
+// corrected solves keep the diagonal blocks T_jj beside their inverses: W(r,
+// c) at [r BF_LD + c] for c <= r, T(r, c) at [c BF_LD + r] for c < r, T(r, r)
+// at [r BF_LD + 16], and a zero that stands for the other halves.
+template <int NB>
+constexpr bool TRSM_FIX = NB <= SMALL_MAX / 16;
+constexpr int TRSM_FIX_ZERO = BF_BLK;
+template <int NB>
+constexpr int TRSM_BLK = TRSM_FIX<NB> ? BF_BLK + 2 : BF_BLK;  // doubles of such a block
+
 // column li of the inverse of a lower 16 x 16 block, lane li holding row li in
-// x and 1 / its diagonal in rd: row C to W[C * BF_LD]
-template <int C>
-__device__ __forceinline__ void tri_inv16(double (&z)[16], const double (&x)[16], double rd,
+// x and 1 / its diagonal in rd: row C to W[C * BF_LD] (FIX: above the
+// diagonal x instead)
+template <bool FIX, int C>
+__device__ __forceinline__ void tri_inv16(double (&z)[16], const double (&x)[16], double rd, int li,
                                           double *W)
 {
     if constexpr (C < 16) {
         z[C] *= bcast16<C>(rd);
-        W[C * BF_LD] = z[C];
+        W[C * BF_LD] = FIX && C < li ? x[C] : z[C];
         fms_lane<C + 1>(z, x[C], z[C]);
-        tri_inv16<C + 1>(z, x, rd, W);
+        tri_inv16<FIX, C + 1>(z, x, rd, li, W);
     }
+}
+
+// The inverses of the diagonal blocks in LDS, and (FIX) the blocks: lane li of
+// a group holds row li in x, its diagonal entry in dv (1: a unit triangle's or
+// a row past the end).
+template <int NB>
+__device__ __forceinline__ void trsm_invert(const double (&x)[16], double dv, int li, double *blk)
+{
+    double v[16];
+#pragma unroll
+    for (int c = 0; c < 16; c++)
+        v[c] = c == li ? 1.0 : 0.0;
+    if (TRSM_FIX<NB>) {
+        blk[li * BF_LD + 16] = dv;
+        blk[TRSM_FIX_ZERO] = 0.0;
+    }
+    tri_inv16<TRSM_FIX<NB>, 0>(v, x, 1.0 / dv, li, blk + li);
+}
+
+// This lane's MFMA A operands from block j of `blk`: element (li, 4 e + lk) of
+// the inverse and (FIX) of the block.
+template <int NB>
+struct TrsmFrag {
+    const double *blk;
+    int ow[4], ot[4];
+    __device__ __forceinline__ TrsmFrag(const double *smem, int li, int lk)
+        : blk(TRSM_FIX<NB> ? smem : smem + li * BF_LD + lk)
+    {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int k = 4 * e + lk;
+            ow[e] = !TRSM_FIX<NB> ? 4 * e : k > li ? TRSM_FIX_ZERO : li * BF_LD + k;
+            ot[e] = k < li ? k * BF_LD + li : k == li ? li * BF_LD + 16 : TRSM_FIX_ZERO;
+        }
+    }
+    __device__ __forceinline__ void load(int j, double (&w)[4], double (&t)[4]) const
+    {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            w[e] = blk[j * TRSM_BLK<NB> + ow[e]];
+            if constexpr (TRSM_FIX<NB>)
+                t[e] = blk[j * TRSM_BLK<NB> + ot[e]];
+        }
+    }
+};
+
+// X_jj = inv(T_jj) Y_j.
+template <int NB>
+__device__ __forceinline__ v4d trsm_diag(const v4d &y, const double (&w)[4], const double (&t)[4])
+{
+    v4d X[1];
+    const v4d Y[1] = {y};
+    if constexpr (TRSM_FIX<NB>) {
+        solve_blk16(X, Y, w, t);
+    } else {
+        X[0] = v4d{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            X[0] = mfma_f64(w[e], Y[0][e], X[0]);
+    }
+    return X[0];
 }
 
 // The T blocks below the diagonal in the order of use, column by column:
@@ -1974,9 +2050,9 @@ __device__ __forceinline__ void trsm_below(v4d (&Y)[NB], const double *ring, con
 // (rlast: the rows below this lane's first that are inside) were updated with
 // rows of T that are not its own; they are zero as its inverse meets them.
 template <int NB, int J>
-__device__ __forceinline__ void trsm_columns(v4d (&Y)[NB], const double *W, const double *ring,
-                                             const int (&lo)[4], int nb, int rlast,
-                                             TrsmFeed<NB> &feed)
+__device__ __forceinline__ void trsm_columns(v4d (&Y)[NB], const TrsmFrag<NB> &frag,
+                                             const double *ring, const int (&lo)[4], int nb,
+                                             int rlast, TrsmFeed<NB> &feed)
 {
     if constexpr (J < NB) {
         if (J >= nb)
@@ -1985,16 +2061,14 @@ __device__ __forceinline__ void trsm_columns(v4d (&Y)[NB], const double *W, cons
 #pragma unroll
             for (int e = 0; e < 4; e++)
                 Y[J][e] = 4 * e < rlast ? Y[J][e] : 0.0;
-        v4d x = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-            x = mfma_f64(W[J * BF_BLK + 4 * e], Y[J][e], x);
-        Y[J] = x;
+        double w[4], t[4];
+        frag.load(J, w, t);
+        Y[J] = trsm_diag<NB>(Y[J], w, t);
         if (J + 1 < nb) {
-            const v4d nx = -x;
+            const v4d nx = -Y[J];
             trsm_below<NB, J, J + 1>(Y, ring, lo, nx, feed);
         }
-        trsm_columns<NB, J + 1>(Y, W, ring, lo, nb, rlast, feed);
+        trsm_columns<NB, J + 1>(Y, frag, ring, lo, nb, rlast, feed);
     }
 }
 
@@ -2013,7 +2087,7 @@ __device__ __attribute__((always_inline)) inline void trsm_panel_reg(const UnitD
     const MU_G double *t = gp(uniform_ptr(u.a));
     MU_G double *z = gp(uniform_ptr(u.c));
     const double alpha = u.alpha;
-    double *ring = smem + NB * BF_BLK;
+    double *ring = smem + NB * TRSM_BLK<NB>;
     // T(r, c) at t[r rs + c cs], Z(r, c) at z[r zrs + c zcs], rows (and T's
     // columns) counted from the end with rev
     const unsigned rs = tt ? ldt : 1, cs = tt ? 1 : ldt;
@@ -2031,7 +2105,7 @@ __device__ __attribute__((always_inline)) inline void trsm_panel_reg(const UnitD
     {
         const int jb = min(wave + 4 * lk, nb - 1);
         const int r = 16 * jb + li, rc = min(r, n - 1);
-        double x[16], v[16];
+        double x[16];
         auto at = [&](int rr, int cc) -> double {
             const size_t a = rev ? n - 1 - rr : rr, b = rev ? n - 1 - cc : cc;
             return t[a * rs + b * cs];
@@ -2041,12 +2115,9 @@ __device__ __attribute__((always_inline)) inline void trsm_panel_reg(const UnitD
             x[c] = at(rc, min(16 * jb + c, n - 1));
         const double dv = at(rc, rc);
 #pragma unroll
-        for (int c = 0; c < 16; c++) {
+        for (int c = 0; c < 16; c++)
             x[c] = r < n ? x[c] : 0.0;
-            v[c] = c == li ? 1.0 : 0.0;
-        }
-        const double rd = ((flags & F_UNIT) || r >= n) ? 1.0 : 1.0 / dv;
-        tri_inv16<0>(v, x, rd, smem + jb * BF_BLK + li);
+        trsm_invert<NB>(x, ((flags & F_UNIT) || r >= n) ? 1.0 : dv, li, smem + jb * TRSM_BLK<NB>);
     }
 
     // ---- the panel (rows past n: the last row).  A wave without right-hand
@@ -2091,7 +2162,8 @@ __device__ __attribute__((always_inline)) inline void trsm_panel_reg(const UnitD
         const int r = rev ? 15 - li : li, c = rev ? 15 - 4 * e - lk : 4 * e + lk;
         lo[e] = tt ? r * 16 + (((c >> 1) ^ ((r >> 1) & 7)) << 1) + (c & 1) : c * 16 + r;
     }
-    trsm_columns<NB, 0>(Y, smem + li * BF_LD + lk, ring, lo, nb, nlast - lk, feed);
+    const TrsmFrag<NB> frag(smem, li, lk);
+    trsm_columns<NB, 0>(Y, frag, ring, lo, nb, nlast - lk, feed);
 
     if (li < w)
 #pragma unroll
@@ -2125,7 +2197,7 @@ __device__ __attribute__((always_inline)) inline void trsm_panel_reg(const UnitD
 // elements take the same updates in the same order, so the results are those
 // of trsm_panel_reg to the bit.  Order 250, one panel: 39 -> 19 us (8.5 us of
 // it the chain: 1400 cycles a step, 1000 where a wave has two rows), order 125
-// 14.5 -> 11 us; LU solve n = 12000, 16 right-hand sides, 5.17 -> 3.16 ms.
+// 17 -> 13 us; LU solve n = 12000, 16 right-hand sides, 5.17 -> 3.16 ms.
 //
 // T is read straight into the MFMA operand by the wave that uses it,
 // TRSM_SPLIT_AHEAD columns ahead.  Nothing but the two products, the LDS
@@ -2146,7 +2218,8 @@ struct TrsmSplit {
     long long step;            // bytes to the next column
     int nb, wave;
     v2d *xb;                   // this lane's part of -X_j, two buffers of 256 doubles
-    v4d Y[NS], W[NS], T[TRSM_SPLIT_AHEAD][NS];
+    v4d Y[NS], T[TRSM_SPLIT_AHEAD][NS];
+    double W[NS][4], D[NS][4];  // the inverse, and the block itself (4 NS blocks at most SMALL_MAX)
 
     // T's column j into d, slots K0 .. (slots above the diagonal read the
     // other triangle and are never used); then on to column j + 1, which
@@ -2179,10 +2252,7 @@ struct TrsmSplit {
 #pragma unroll
             for (int e = 0; e < 4; e++)
                 y[e] = 4 * e < rlast ? y[e] : 0.0;
-        v4d x = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-            x = mfma_f64(W[J / 4][e], y[e], x);
+        const v4d x = trsm_diag<4 * NS>(y, W[J / 4], D[J / 4]);
         y = x;
         v2d *o = xb + (J & 1) * 128;
         o[0] = v2d{-x[0], -x[1]};
@@ -2251,11 +2321,12 @@ __device__ __attribute__((always_inline)) inline void trsm_panel_split(const Uni
     TrsmSplit<NS> p;
     p.nb = nb;
     p.wave = wave;
-    p.xb = reinterpret_cast<v2d *>(smem + 4 * NS * BF_BLK) + lane;
+    constexpr int BLK = TRSM_BLK<4 * NS>;
+    p.xb = reinterpret_cast<v2d *>(smem + 4 * NS * BLK) + lane;
 
     // ---- the diagonal blocks, block wave + 4 lk on this group
     const int jb = min(wave + 4 * lk, nb - 1), r = 16 * jb + li, rc = min(r, n - 1);
-    double x[16], v[16];
+    double x[16];
     {
         // rows past n: the last one; columns past n: the last one
         const size_t a = (size_t)(rev ? n - 1 - rc : rc) * rs;
@@ -2306,21 +2377,17 @@ __device__ __attribute__((always_inline)) inline void trsm_panel_split(const Uni
 
     // ---- the inverses; a wave reads back those of its own rows
 #pragma unroll
-    for (int c = 0; c < 16; c++) {
+    for (int c = 0; c < 16; c++)
         x[c] = r < n ? x[c] : 0.0;
-        v[c] = c == li ? 1.0 : 0.0;
-    }
-    const double rd = ((flags & F_UNIT) || r >= n) ? 1.0 : 1.0 / dv;
-    tri_inv16<0>(v, x, rd, smem + jb * BF_BLK + li);
+    trsm_invert<4 * NS>(x, ((flags & F_UNIT) || r >= n) ? 1.0 : dv, li, smem + jb * BLK);
+    const TrsmFrag<4 * NS> frag(smem, li, lk);
     lds_barrier();  // the last block's inverse may have been formed by every wave
 #pragma unroll
     for (int k = 0; k < NS; k++) {
-        const double *b = smem + min(4 * k + wave, nb - 1) * BF_BLK + li * BF_LD + lk;
+        frag.load(min(4 * k + wave, nb - 1), p.W[k], p.D[k]);
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            p.W[k][e] = b[4 * e];
+        for (int e = 0; e < 4; e++)
             p.Y[k][e] *= alpha;
-        }
     }
 
     if (wave == 0)
@@ -2340,7 +2407,7 @@ __device__ __attribute__((always_inline)) inline void trsm_panel_split(const Uni
 }
 
 constexpr int LDS_TRSM_REG = 16 * BF_BLK + TRSM_RING<16> * 1024;       // inverses of order TRSM_REG_MAX
-constexpr int LDS_TRSM_REG_SMALL = 8 * BF_BLK + TRSM_RING<8> * 1024;  // ... of order SMALL_MAX
+constexpr int LDS_TRSM_REG_SMALL = 8 * TRSM_BLK<8> + TRSM_RING<8> * 1024;  // ... of order SMALL_MAX
 
 // TRSM item of a triangle of order <= TRSM_REG_MAX; MAXNB: the most 16-blocks
 // the caller's LDS holds inverses for (8 or 16).  The block count is rounded
