@@ -1360,9 +1360,43 @@ __device__ __forceinline__ void update_row(v4d *acc, const double *lds, const v4
 // instructions on the vector ALU, each of which waits behind the MFMAs of the
 // GEMM workgroups on its SIMD.  Order 128 in a graph node: POTRF 29.0 -> 32.2
 // us, GETRF 39.0 -> 46.9 us (1.9 of these for getrf16's consistent factors).
+//
+// A column that is not finite afterwards is substituted: the products multiply
+// the other halves' zeros too, and would spread a NaN or an infinity to the
+// rows before it.  `tri` is the triangle in LDS.  A column's first rows show it:
+// 0 * inf and 0 * NaN are NaN.
+__device__ __forceinline__ const MU_LDS double *lp(const double *p)
+{
+    return (const MU_LDS double *)p;
+}
+
+struct TriRef {
+    const MU_LDS double *t;  // T(r, c) at t[r rs + c cs], c < r
+    int rs, cs;
+    const MU_LDS double *d;  // 1 / T(r, r) at d[r (BF_LD + 1)]: the inverse's diagonal
+};
+
+// Y = inv(T) Y by substitution.
+__device__ __noinline__ inline v4d subst_blk16(v4d y, TriRef tri)
+{
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+#pragma unroll 1
+    for (int r = 0; r < 16; r++) {
+        double v = r < 4 ? y[0] : r < 8 ? y[1] : r < 12 ? y[2] : y[3];
+        v = __shfl(v, li + 16 * (r & 3)) * tri.d[r * (BF_LD + 1)];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int i = 4 * e + lk;
+            const double f = fma(-tri.t[i * tri.rs + r * tri.cs], v, y[e]);
+            y[e] = i == r ? v : i > r ? f : y[e];
+        }
+    }
+    return y;
+}
+
 template <int N>
 __device__ __forceinline__ void solve_blk16(v4d (&X)[N], const v4d (&Y)[N], const double (&w)[4],
-                                            const double (&t)[4])
+                                            const double (&t)[4], const TriRef &tri)
 {
     v4d R[N];
 #pragma unroll
@@ -1385,6 +1419,21 @@ __device__ __forceinline__ void solve_blk16(v4d (&X)[N], const v4d (&Y)[N], cons
 #pragma unroll
         for (int b = 0; b < N; b++)
             X[b] = mfma_f64(w[e], R[b][e], X[b]);
+    unsigned long long bad[N], any = 0;
+#pragma unroll
+    for (int b = 0; b < N; b++) {
+        bad[b] = __ballot(!(fabs(X[b][0]) < __builtin_inf()));
+        any |= bad[b];
+    }
+    if (__builtin_expect(any != 0, 0)) {
+        const int li = threadIdx.x & 15;
+#pragma unroll
+        for (int b = 0; b < N; b++) {
+            const v4d y = subst_blk16(Y[b], tri);
+            const unsigned long long m = bad[b] | bad[b] >> 32, col = (m | m >> 16) >> li;
+            X[b] = col & 1 ? y : X[b];
+        }
+    }
 }
 
 struct SmallCtx {
@@ -1478,6 +1527,7 @@ __device__ __forceinline__ void potrf_step(const SmallCtx &c, v4d (&R0)[4], v4d 
     const bool on1 = c.w + 4 > P && c.w + 4 < c.nb;
     v4d X0, X1;
     double wv[4], tv[4];
+    const TriRef tri = {lp(D), BF_LD, 1, lp(W)};
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         const int k = 4 * e + c.lk;
@@ -1488,7 +1538,7 @@ __device__ __forceinline__ void potrf_step(const SmallCtx &c, v4d (&R0)[4], v4d 
         if (on0) {  // row w + 4 may be past the tile: a block nothing reads
             v4d X[2];
             const v4d Y[2] = {R0[P], R1[P]};
-            solve_blk16(X, Y, wv, tv);
+            solve_blk16(X, Y, wv, tv, tri);
             X0 = X[0];
             X1 = X[1];
         }
@@ -1496,7 +1546,7 @@ __device__ __forceinline__ void potrf_step(const SmallCtx &c, v4d (&R0)[4], v4d 
     if (!on0 && on1) {
         v4d X[1];
         const v4d Y[1] = {R1[P]};
-        solve_blk16(X, Y, wv, tv);
+        solve_blk16(X, Y, wv, tv, tri);
         X1 = X[0];
     }
     auto put = [&](int i, const v4d &x) {
@@ -1667,6 +1717,7 @@ __device__ __forceinline__ void getrf_step(const SmallCtx &c, v4d (&R0)[8], v4d 
     const bool on1 = c.w + 4 > P && c.w + 4 < c.nb;
     v4d X0, X1;
     double wv[4], tv[4];
+    const TriRef ut = {lp(D), 1, BF_LD, lp(W2)}, l = {lp(D), BF_LD, 1, lp(W1)};
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         const int k = 4 * e + c.lk;
@@ -1677,7 +1728,7 @@ __device__ __forceinline__ void getrf_step(const SmallCtx &c, v4d (&R0)[8], v4d 
         if (on0) {  // row w + 4 may be past the tile: a block nothing reads
             v4d X[2];
             const v4d Y[2] = {R0[P], R1[P]};
-            solve_blk16(X, Y, wv, tv);
+            solve_blk16(X, Y, wv, tv, ut);
             X0 = X[0];
             X1 = X[1];
         }
@@ -1685,7 +1736,7 @@ __device__ __forceinline__ void getrf_step(const SmallCtx &c, v4d (&R0)[8], v4d 
     if (!on0 && on1) {
         v4d X[1];
         const v4d Y[1] = {R1[P]};
-        solve_blk16(X, Y, wv, tv);
+        solve_blk16(X, Y, wv, tv, ut);
         X1 = X[0];
     }
     if (P + 1 + c.w < c.nb) {
@@ -1701,7 +1752,7 @@ __device__ __forceinline__ void getrf_step(const SmallCtx &c, v4d (&R0)[8], v4d 
 #pragma unroll
             for (int e = 0; e < 4; e++)
                 Y[0][e] = b[(4 * e + c.lk) * BF_LD + c.li];
-            solve_blk16(X, Y, wv, tv);
+            solve_blk16(X, Y, wv, tv, l);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 Ub[(j - 1) * 256 + e * 64 + c.lane] = -X[0][e];
@@ -1949,14 +2000,15 @@ struct TrsmFrag {
     }
 };
 
-// X_jj = inv(T_jj) Y_j.
+// X_j = inv(T_jj) Y_j; `blk` is block j (FIX).
 template <int NB>
-__device__ __forceinline__ v4d trsm_diag(const v4d &y, const double (&w)[4], const double (&t)[4])
+__device__ __forceinline__ v4d trsm_diag(const v4d &y, const double (&w)[4], const double (&t)[4],
+                                         const double *blk)
 {
     v4d X[1];
     const v4d Y[1] = {y};
     if constexpr (TRSM_FIX<NB>) {
-        solve_blk16(X, Y, w, t);
+        solve_blk16(X, Y, w, t, TriRef{lp(blk), 1, BF_LD, lp(blk)});
     } else {
         X[0] = v4d{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
@@ -2063,7 +2115,7 @@ __device__ __forceinline__ void trsm_columns(v4d (&Y)[NB], const TrsmFrag<NB> &f
                 Y[J][e] = 4 * e < rlast ? Y[J][e] : 0.0;
         double w[4], t[4];
         frag.load(J, w, t);
-        Y[J] = trsm_diag<NB>(Y[J], w, t);
+        Y[J] = trsm_diag<NB>(Y[J], w, t, frag.blk + J * TRSM_BLK<NB>);
         if (J + 1 < nb) {
             const v4d nx = -Y[J];
             trsm_below<NB, J, J + 1>(Y, ring, lo, nx, feed);
@@ -2217,6 +2269,7 @@ struct TrsmSplit {
     unsigned tl[4], tlast[4];  // this lane's byte offset of element e, and in the last slot
     long long step;            // bytes to the next column
     int nb, wave;
+    const double *blk;         // the diagonal blocks and their inverses
     v2d *xb;                   // this lane's part of -X_j, two buffers of 256 doubles
     v4d Y[NS], T[TRSM_SPLIT_AHEAD][NS];
     double W[NS][4], D[NS][4];  // the inverse, and the block itself (4 NS blocks at most SMALL_MAX)
@@ -2252,7 +2305,7 @@ struct TrsmSplit {
 #pragma unroll
             for (int e = 0; e < 4; e++)
                 y[e] = 4 * e < rlast ? y[e] : 0.0;
-        const v4d x = trsm_diag<4 * NS>(y, W[J / 4], D[J / 4]);
+        const v4d x = trsm_diag<4 * NS>(y, W[J / 4], D[J / 4], blk + J * TRSM_BLK<4 * NS>);
         y = x;
         v2d *o = xb + (J & 1) * 128;
         o[0] = v2d{-x[0], -x[1]};
@@ -2322,6 +2375,7 @@ __device__ __attribute__((always_inline)) inline void trsm_panel_split(const Uni
     p.nb = nb;
     p.wave = wave;
     constexpr int BLK = TRSM_BLK<4 * NS>;
+    p.blk = smem;
     p.xb = reinterpret_cast<v2d *>(smem + 4 * NS * BLK) + lane;
 
     // ---- the diagonal blocks, block wave + 4 lk on this group
