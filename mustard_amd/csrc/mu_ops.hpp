@@ -78,17 +78,28 @@ constexpr int LDS_K = GEMM_BM * PK;   // doubles per k-contiguous buffer
 // into the operand; the values that fall outside it are zeroed only when the
 // registers are written to LDS.  With no branch around a load and no use of
 // its result before the LDS store, the compiler's wait counting stays exact
-// and a prefetch stays in flight until the half-step that stores it.
+// and a prefetch stays in flight until the half-step that stores it.  VEC
+// (16-byte aligned operands, even leading dimensions and even m, n, k, set by
+// the lowering) loads element pairs, which then never straddle an edge: 4000 x
+// 32 x 1000 in 57 us against 62.
 
 // i-contiguous operand: element (r, k) at p[r + k*ld], r < rows, k < kcols.
 // Thread t covers rows 2(t%32), 2(t%32)+1 of column t/32.
+template <bool VEC>
 __device__ __forceinline__ void ld_icontig(double (&v)[2], const MU_G double *p, int ld, int rows,
                                            int kcols)
 {
     const int t = threadIdx.x, r = (t & 31) * 2, c = t >> 5;
     const int cc = max(0, min(c, kcols - 1));
-    v[0] = p[min(r, rows - 1) + (size_t)cc * ld];
-    v[1] = p[min(r + 1, rows - 1) + (size_t)cc * ld];
+    if (VEC) {
+        const int rr = max(0, min(r, rows - 2));
+        const v2d x = *reinterpret_cast<const MU_G v2d *>(p + rr + (size_t)cc * ld);
+        v[0] = x[0];
+        v[1] = x[1];
+    } else {
+        v[0] = p[min(r, rows - 1) + (size_t)cc * ld];
+        v[1] = p[min(r + 1, rows - 1) + (size_t)cc * ld];
+    }
 }
 
 __device__ __forceinline__ void st_icontig(double *S, const double (&v)[2], int rows, int kcols)
@@ -103,13 +114,21 @@ __device__ __forceinline__ void st_icontig(double *S, const double (&v)[2], int 
 
 // k-contiguous operand: element (r, k) at p[k + r*ld].
 // Thread t covers k = 2(t%4), 2(t%4)+1 of row t/4.
+template <bool VEC>
 __device__ __forceinline__ void ld_kcontig(double (&v)[2], const MU_G double *p, int ld, int rows,
                                            int kcols)
 {
     const int t = threadIdx.x, k = (t & 3) * 2, r = t >> 2;
     const int rr = min(r, rows - 1);
-    v[0] = p[max(0, min(k, kcols - 1)) + (size_t)rr * ld];
-    v[1] = p[max(0, min(k + 1, kcols - 1)) + (size_t)rr * ld];
+    if (VEC) {
+        const int kk = max(0, min(k, kcols - 2));
+        const v2d x = *reinterpret_cast<const MU_G v2d *>(p + kk + (size_t)rr * ld);
+        v[0] = x[0];
+        v[1] = x[1];
+    } else {
+        v[0] = p[max(0, min(k, kcols - 1)) + (size_t)rr * ld];
+        v[1] = p[max(0, min(k + 1, kcols - 1)) + (size_t)rr * ld];
+    }
 }
 
 __device__ __forceinline__ void st_kcontig(double *S, const double (&v)[2], int rows, int kcols)
@@ -134,7 +153,7 @@ __device__ __forceinline__ double frag_b(const double *S, int k, int j)
     return TB ? S[k * PI + j] : S[j * PK + k];
 }
 
-template <bool TA, bool TB>
+template <bool TA, bool TB, bool VEC>
 __device__ __attribute__((always_inline)) inline void gemm_block(const UnitDesc &u, int bi, int bj, bool lower_only, double *smem)
 {
     constexpr int BM = GEMM_BM, BN = GEMM_BN, BK = GEMM_BK;
@@ -165,13 +184,13 @@ __device__ __attribute__((always_inline)) inline void gemm_block(const UnitDesc 
         // a block past K is read (and zeroed) at k-offset 0, inside the operand
         const int kc = K - k0, ks = kc > 0 ? k0 : 0;
         if (TA)
-            ld_kcontig(ra, A + ks, u.lda, rows, kc);
+            ld_kcontig<VEC>(ra, A + ks, u.lda, rows, kc);
         else
-            ld_icontig(ra, A + (size_t)ks * u.lda, u.lda, rows, kc);
+            ld_icontig<VEC>(ra, A + (size_t)ks * u.lda, u.lda, rows, kc);
         if (TB)
-            ld_icontig(rb, B + (size_t)ks * u.ldb, u.ldb, cols, kc);
+            ld_icontig<VEC>(rb, B + (size_t)ks * u.ldb, u.ldb, cols, kc);
         else
-            ld_kcontig(rb, B + ks, u.ldb, cols, kc);
+            ld_kcontig<VEC>(rb, B + ks, u.ldb, cols, kc);
     };
     // store the block loaded for k-offset k0 (zeroing what lies outside)
     auto store = [&](const double (&ra)[2], const double (&rb)[2], double *As, double *Bs,
@@ -2586,7 +2605,10 @@ __device__ __forceinline__ void gemm_dispatch_vec(const UnitDesc &u, int bi, int
     } else if (gemm_dma_ok(u)) {
         gemm_block_dma<TA, TB>(u, bi, bj, lo, smem);
     } else {
-        gemm_block<TA, TB>(u, bi, bj, lo, smem);
+        if (u.flags & F_VEC)
+            gemm_block<TA, TB, true>(u, bi, bj, lo, smem);
+        else
+            gemm_block<TA, TB, false>(u, bi, bj, lo, smem);
     }
 }
 
