@@ -242,8 +242,10 @@ __global__ void k_fill_u64(unsigned long long *p, int n, unsigned long long v)
 // (a wave reads 64 consecutive rows of a column, 16 loads in flight), and
 // BRES_WGS workgroups share a problem; with one workgroup per problem and a
 // thread per row, the largest problem's rows were one serial chain of n
-// loads (288 problems of order 32..1024: 1660 -> 103 us).  A row's four partial sums
-// are added in a fixed order.  Maxima on the bit patterns of non-negative
+// loads (288 problems of order 32..1024: 1660 -> 94 us).  With 4 / 8 / 16 / 32
+// workgroups a problem, 32 problems take 35 / 26 / 18 / 21 us, 288 take 119 / 107
+// / 94 / 151 us and 2000 take 475 / 445 / 547 / 900 us.  A row's four partial
+// sums are added in a fixed order.  Maxima on the bit patterns of non-negative
 // values (a NaN's pattern sorts above inf, so NaN propagates).
 constexpr int BRES_WGS = 16;
 
