@@ -45,7 +45,9 @@ typedef struct mu_exec_s *mu_exec_t;
 typedef struct {
     int grid;           /* persistent grid size, 0 = one workgroup per CU slot */
     double timeout_s;   /* persistent: abort after this long without progress (0 = 10 s);
-                           a host watchdog aborts a run after 3 * timeout_s + 1 s */
+                           a host watchdog aborts a run after 3 * timeout_s + 1 s: a
+                           waiting run sees that within about a millisecond, a busy one
+                           after about as many items as it has workgroups */
     int trace;          /* persistent: record per-item wall-clock stamps */
     int small_max;      /* diagonal factorizations above this order nest (0 = 128) */
     int trsm_max;       /* triangular solves above this order nest (0 = 256; at most 1024) */
@@ -131,7 +133,7 @@ int mu_dtrsm(void *stream, char side, char uplo, char transa, char diag, int m, 
  * (bit for bit), run at once on `stream`.  Triangles of order <= 8192 are
  * accepted and larger ones rejected with MU_EINVAL; a stream being recorded
  * into a DAG is refused (MU_ESTATE).  Allocates no device memory and keeps
- * none (MU_NOALLOC_SCRATCH_BYTES, the size of a device array that earlier
+ * none, so calls on different streams may overlap (MU_NOALLOC_SCRATCH_BYTES, the size of a device array that earlier
  * versions held, is defined for callers that read it). */
 #define MU_NOALLOC_SCRATCH_BYTES (1u << 21)
 #define MU_NOALLOC_MAX_ORDER 8192
@@ -285,8 +287,8 @@ int mu_record_batch(mu_dag_t dag, int nprob, const int *kinds, const int *ns, do
  * order of problem p, a_off[p] the element offset of its n x n matrix
  * (leading dimension n) in A, v_off[p] the offset of its vectors in X, B and
  * R.  Writes r_p = b_p - A_p x_p (FP64) to R and, per problem, norms[4p..4p+3]
- * = ||r||_inf, ||x||_inf, ||A||_inf, ||b||_inf (NaN propagates).  One
- * workgroup per problem, one launch. */
+ * = ||r||_inf, ||x||_inf, ||A||_inf, ||b||_inf (NaN propagates).  R and
+ * norms overlap none of the inputs. */
 int mu_batch_residual(int nprob, const int *ns, const long long *a_off, const long long *v_off,
                       const double *A, const double *X, const double *B, double *R,
                       double *norms, void *stream);

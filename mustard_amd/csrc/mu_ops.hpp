@@ -865,7 +865,7 @@ constexpr int LDS_GEMM_LOWK128 = 2 * 256 * (64 + 8) * 2 / 8;
 // ---------------------------------------------------------------------------
 // Inverted diagonal blocks.  For a triangle T of order n > TRSM_REG_MAX (read in
 // the canonical lower form the panel solve uses: flags TT, UNIT, REV as in
-// trsm_panel), item `it` inverts diagonal blocks 16*it .. 16*it+15 of 16 x 16
+// trsm_panel_inv), item `it` inverts diagonal blocks 16*it .. 16*it+15 of 16 x 16
 // and stores inv(T_jj) row-major at c + 256 j.  Rows and columns of the last
 // block past n are the identity.  Thread t: block t/16, column t%16, by
 // forward substitution against the unit vector (divisions, as LAPACK's
@@ -923,10 +923,10 @@ __device__ __attribute__((always_inline)) inline void trinv_blocks(const UnitDes
 // Panel triangular solve in LDS with inverted diagonal blocks (triangles of
 // order n > TRSM_REG_MAX, made only where mu_exec_opts_t.trsm_max asks for
 // them; the TRINV unit before it left inv(T_jj) at u.b).  Same problem and
-// flags as trsm_panel_reg, panels of 16 right-hand sides.  Step jb: every wave forms the solved
-// block X_jb = inv(T_jj) Y_jb with four MFMAs -- the result's register layout
-// is exactly the B operand of the update MFMAs, so it never goes back
-// through LDS -- wave 0 stores it to Z, and each wave updates its row blocks
+// flags as trsm_panel_reg, panels of 16 right-hand sides.  Step jb: every wave
+// forms the solved block X_jb = inv(T_jj) Y_jb with four MFMAs -- the result's
+// register layout is exactly the B operand of the update MFMAs, so it never
+// goes back through LDS -- wave 0 stores it to Z, and each wave updates its row blocks
 // below, Y[rb] -= T[rb, jb] X_jb.  One barrier per step.  The next step's
 // inverse block and triangle fragments are loaded during the current step
 // (the latter row block by row block, right after that block's MFMAs).
@@ -3079,8 +3079,7 @@ __device__ __attribute__((always_inline)) inline void run_trinv_item(const UnitD
     }
 }
 
-// Small GETRF/POTRF or CVT item (the only kinds k_batch_small runs), on NW
-// waves; a CVT item uses the first four.
+// Small GETRF/POTRF or CVT item (the only kinds k_batch_small runs).
 __device__ __attribute__((always_inline)) inline void run_small_item(const UnitDesc &u, int it,
                                                                      double *smem)
 {

@@ -30,7 +30,7 @@ enum Op : int32_t {
 enum Flag : int32_t {
     F_TA = 1 << 0,       // GEMM: op(A) = A^T
     F_TB = 1 << 1,       // GEMM: op(B) = B^T
-    F_VEC = 1 << 2,      // operands 16-byte aligned with even leading dims: vector loads
+    F_VEC = 1 << 2,      // operands 16-byte aligned with even leading dims and sizes: vector loads
     F_T_TRANS = 1 << 3,  // TRSM: triangle read transposed, T[r][c] = t[c + r*ldt]
     F_Z_ROWS = 1 << 4,   // TRSM: right-hand sides are rows, Z[r][c] = z[c + r*ldz]
     F_UNIT = 1 << 5,     // TRSM: unit diagonal
