@@ -1369,33 +1369,20 @@ __device__ __forceinline__ void update_row(v4d *acc, const double *lds, const v4
     }
 }
 
-// X = inv(T) Y for N blocks of Y in register format, T a lower 16 x 16
-// triangle: W ~ inv(T) and T come as this lane's MFMA A operands, element
-// (li, 4 e + lk).  The product with an inverse alone leaves a residual of eps
-// cond(T) where substitution leaves eps -- a Cholesky of a kernel matrix (128
-// points, 1e-12 added to the diagonal) then met a negative pivot -- so it is
-// corrected once, X += W (Y - T X): the residual falls to eps + (eps
-// cond(T))^2.  That is eight more MFMAs per block; substitution is 136
-// instructions on the vector ALU, each of which waits behind the MFMAs of the
-// GEMM workgroups on its SIMD.  Order 128 in a graph node: POTRF 29.0 -> 32.2
-// us, GETRF 39.0 -> 46.9 us (1.9 of these for getrf16's consistent factors).
-//
-// A column that is not finite afterwards is substituted: the products multiply
-// the other halves' zeros too, and would spread a NaN or an infinity to the
-// rows before it.  `tri` is the triangle in LDS.  A column's first rows show it:
-// 0 * inf and 0 * NaN are NaN.
 __device__ __forceinline__ const MU_LDS double *lp(const double *p)
 {
     return (const MU_LDS double *)p;
 }
 
+// A lower 16 x 16 triangle in LDS.
 struct TriRef {
     const MU_LDS double *t;  // T(r, c) at t[r rs + c cs], c < r
     int rs, cs;
     const MU_LDS double *d;  // 1 / T(r, r) at d[r (BF_LD + 1)]: the inverse's diagonal
 };
 
-// Y = inv(T) Y by substitution.
+// inv(T) Y by substitution, out of line: the kernels that call it keep their
+// size and registers (inlined at its 48 places it doubles k_batch_small).
 __device__ __noinline__ inline v4d subst_blk16(v4d y, TriRef tri)
 {
     const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
@@ -1413,6 +1400,21 @@ __device__ __noinline__ inline v4d subst_blk16(v4d y, TriRef tri)
     return y;
 }
 
+// X = inv(T) Y for N blocks of Y in register format, T a lower 16 x 16
+// triangle: W ~ inv(T) and T come as this lane's MFMA A operands, element
+// (li, 4 e + lk).  The product with an inverse alone leaves a residual of eps
+// cond(T) where substitution leaves eps -- a Cholesky of a kernel matrix (128
+// points, 1e-12 added to the diagonal) then met a negative pivot -- so it is
+// corrected once, X += W (Y - T X): the residual falls to eps + (eps
+// cond(T))^2.  That is eight more MFMAs per block; substitution is 136
+// instructions on the vector ALU, each of which waits behind the MFMAs of the
+// GEMM workgroups on its SIMD.  Order 128 in a graph node: POTRF 29.0 -> 32.2
+// us, GETRF 39.0 -> 46.9 us (1.9 of these for getrf16's consistent factors).
+//
+// A column that is not finite afterwards is substituted: the products multiply
+// the other halves' zeros too, and would spread a NaN or an infinity to the
+// rows before it.  `tri` is the triangle in LDS.  A column's first rows show it:
+// 0 * inf and 0 * NaN are NaN.
 template <int N>
 __device__ __forceinline__ void solve_blk16(v4d (&X)[N], const v4d (&Y)[N], const double (&w)[4],
                                             const double (&t)[4], const TriRef &tri)
